@@ -8,7 +8,7 @@
 // last n positions (n = position + 1, or at most 1024 for a local ring), read from cache
 // row (first + offset) % cap.
 //
-// Split kernel (k_attn_mx): one wave per (sequence, KV head, split), over that split's
+// Split kernel (k_attn_mx): one workgroup per (sequence, KV head, split), over that split's
 // 32-key tiles, QK and PV on the matrix cores; the reference's online softmax per row
 // (tile maximum, fp32 probabilities for the denominator fmaf(den, alpha, total), BF16
 // probabilities for the PV product, scale 1/sqrt(128) applied after the dot product).
@@ -39,7 +39,7 @@ namespace {
 constexpr int kD = 128, kKeys = 32;
 // Launches of up to this many sequences on a global cache order their split waves by
 // window length (the ranking reads seqs^2 control records).
-constexpr int kOrderMaxSeqs = 512;
+constexpr int kOrderMaxSeqs = 512, kRankMaxSeqs = 64;
 constexpr float kScoreScale = .08838834764831845f;
 
 int launched(const char *what) {
@@ -58,7 +58,7 @@ struct AttnArgs {
   void *out; // [seqs][hq][128]
   float *partial, *lse;
   const padra_DecodeState *decode;
-  int seqs, hq, hkv, cap, local, splits, maximum, vocab;
+  int seqs, hq, hkv, group, cap, local, splits, maximum, vocab;
   long long seq_stride; // cache rows between sequences
   int *bad;
   // q8_0 caches: the coded query (int8 [seqs][hq][128]) and its block scales
@@ -69,6 +69,8 @@ struct AttnArgs {
   // The split kernels' sequence for grid slot z (longest window first), or null for
   // slot z = sequence z.
   int *order;
+  // Each split wave ranks the sequences itself (at most 64 of them, one per lane).
+  int rank;
 };
 
 // The sequence's admission and key window (Admitted, attention_gqa8_fragment_validation.cuh:
@@ -99,8 +101,31 @@ __device__ __forceinline__ void attn_rank(const AttnArgs &a, int seq) {
   if (threadIdx.x == 0)
     a.order[before] = seq;
 }
-__device__ __forceinline__ int attn_seq(const AttnArgs &a) {
-  return a.order ? a.order[blockIdx.z] : (int)blockIdx.z;
+// The split kernels' sequence for grid slot blockIdx.z, its admission and key window.  With
+// a.rank each wave ranks the sequences itself, one a lane: 0.1-0.5 us of its time against
+// a launch of its own for k_attn_order, whose 4.3 us (2 of them not hidden) every step paid.
+__device__ __forceinline__ bool attn_pick(const AttnArgs &a, int &seq, int &n, int &first) {
+  const int slot = blockIdx.z;
+  if (!a.rank) {
+    seq = a.order ? __builtin_amdgcn_readfirstlane(a.order[slot]) : slot;
+    return attn_window(a, seq, n, first);
+  }
+  const int lane = threadIdx.x & 63;
+  int mine = 0, from = 0;
+  bool ok = false;
+  if (lane < a.seqs)
+    ok = attn_window(a, lane, mine, from);
+  // window length (0 if not admitted), then the lower index: distinct keys
+  const int key = lane < a.seqs ? ((ok ? mine : 0) << 6) + 63 - lane : -1;
+  int before = 0;
+  for (int j = 0; j < a.seqs; j += 8)
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      before += __builtin_amdgcn_readlane(key, j + i) > key;
+  seq = (int)__builtin_ctzll(__ballot(lane < a.seqs && before == slot));
+  n = __builtin_amdgcn_readlane(mine, seq);
+  first = __builtin_amdgcn_readlane(from, seq);
+  return __builtin_amdgcn_readlane((int)ok, seq) != 0;
 }
 
 __global__ __launch_bounds__(64) void k_attn_order(AttnArgs a) { attn_rank(a, blockIdx.x); }
@@ -136,18 +161,26 @@ template <class T> __device__ __forceinline__ float act_value(const void *p, siz
 
 // ---- Split kernel on the matrix cores --------------------------------------------------
 // QK and PV on v_mfma_f32_16x16x32_bf16 (the reference runs both on tensor-core MMA).  One
-// wave per (sequence, KV head, split); query rows are the 16 MFMA columns (rows past G are
-// zero).
-//  - QK: S[key][row] = K[key][:] . Q[row][:] for the tile's two 16-key halves, 4 K-steps of
-//    32 dimensions each.  Lane l then holds row l % 16, keys 16 h + 4 (l / 16) + i.
+// workgroup of W waves per (sequence, KV head, split), over the split's tiles in rounds of W;
+// query rows are the 16 MFMA columns (rows past the group are zero).
+//  - QK, a tile per wave: S[key][row] = K[key][:] . Q[row][:] for the tile's two 16-key halves,
+//    4 K-steps of 32 dimensions each.  Lane l then holds row l % 16, keys 16 h + 4 (l / 16) + i.
 //  - Softmax: the row's tile maximum and probability sum are the lane's 8 values plus two
-//    exchanges between the four lanes of the row.
-//  - PV: O[row][dim] += P[row][key] V[key][dim] with P straight from the score registers
-//    (K-slot i of lane group g is key 4g + i, then 16 + 4g + i - 4) and V staged in LDS as
-//    4-key groups per dimension, so that each B operand is two 8-byte LDS reads.  Lane l
-//    holds rows 4 (l / 16) + i of dimension 16 b + l % 16.
-//  - The accumulators are rescaled only when some row's maximum moved (alpha == 1 exactly
-//    otherwise).
+//    exchanges between the four lanes of the row.  The tile maxima of a round cross LDS, so
+//    that each wave knows the running maximum at its tile: probabilities, rescale factors
+//    and the denominator's terms are those of one wave walking the tiles in order.
+//  - PV, 8 / W blocks of 16 dimensions per wave, over the round's tiles in order: O[row][dim] +=
+//    P[row][key] V[key][dim] with P from the score registers (K-slot i of lane group g is key
+//    4g + i, then 16 + 4g + i - 4) and V staged in LDS as 4-key groups per dimension, so that
+//    each B operand is two 8-byte LDS reads.  Lane l holds rows 4 (l / 16) + i of dimension
+//    16 b + l % 16.  Every sum thus has the order it has with one wave, and the results are
+//    the same bits for every W.
+//
+// What bounds it: with few sequences the bytes in flight (one wave a split: 1.5 TB/s at one
+// sequence of 32768 keys), with many the memory rate (5.9 TB/s at 64; a kernel that only reads
+// reaches 7.0).  Several waves a split give each its tile's 16 KB of loads at once and divide
+// PV: one sequence of 131072 keys 148.9 -> 75.6 us (BF16), 231.5 -> 71.3 us (q8); of 32768 keys
+// 45.9 -> 26.4 and 66.4 -> 26.1 us; 8 sequences to 8000 keys 29.9 -> 25.2 and 31.3 -> 24.3 us.
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
@@ -164,33 +197,39 @@ __device__ __forceinline__ bool q8_scale_fast(float scale) {
   return scale > 0.f && 127.f * scale < 0x1.ffp127f;
 }
 
-// The 16 values code * scale of a code chunk (kv_q8::Decode), with the least code seen
-// (as a float; -128 is the code the reference rejects) and whether the scale passes
-// q8_scale_fast.  The caller gives keys past the window zero codes and a unit scale, as
-// the reference stages them.  Each code is one v_cvt_f32_i32 with a sign-extended byte
-// select.
-__device__ __forceinline__ void q8_values16(uint4 c, float scale, float (&f)[16], float &least,
-                                            bool &slow) {
-  const uint32_t w[4] = {c.x, c.y, c.z, c.w};
-  float code[16];
+// The values code * scale of a word of four codes (kv_q8::Decode), with the least code seen
+// (as a float; -128 is the code the reference rejects).  The caller gives keys past the
+// window zero codes and a unit scale, as the reference stages them.  Each code is one
+// v_cvt_f32_i32 with a sign-extended byte select; min(min(least, a), b) is one v_min3_f32.
+__device__ __forceinline__ void q8_values4(uint32_t w, float scale, float *f, float &least) {
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int b = 0; b < 4; ++b)
+    f[b] = (float)(int8_t)((w >> (8 * b)) & 0xffu);
 #pragma unroll
-    for (int b = 0; b < 4; ++b)
-      code[4 * i + b] = (float)(int8_t)((w[i] >> (8 * b)) & 0xffu);
+  for (int b = 0; b < 4; ++b)
+    least = fminf(least, f[b]);
+  // Here and not where it is used: sunk to there, it kept every code of the tile in
+  // registers (256 VGPRs and more).
+  asm volatile("" : "+v"(least));
 #pragma unroll
-  for (int i = 0; i < 16; ++i) // min(min(least, a), b): one v_min3_f32 per pair
-    least = fminf(least, code[i]);
-#pragma unroll
-  for (int i = 0; i < 16; ++i)
-    f[i] = code[i] * scale;
-  slow = slow || !q8_scale_fast(scale);
+  for (int b = 0; b < 4; ++b)
+    f[b] = f[b] * scale;
+}
+__device__ __forceinline__ void q8_values8(uint32_t w0, uint32_t w1, float scale, float (&f)[8],
+                                           float &least) {
+  q8_values4(w0, scale, f, least);
+  q8_values4(w1, scale, f + 4, least);
 }
 
 // kv_q8::Decode's checks on a chunk whose scale failed q8_scale_fast: a valid scale and
 // every code * scale finite in BF16.
 __device__ __forceinline__ bool q8_check16(uint4 c, float scale) {
-  const uint32_t w[4] = {c.x, c.y, c.z, c.w};
+  uint32_t w[4] = {c.x, c.y, c.z, c.w};
+  // An opaque copy: the compiler would otherwise keep every decoded value of the tile in
+  // registers for this rare path (400 VGPRs).
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    asm volatile("" : "+v"(w[i]));
   bool ok = isfinite(scale) && scale > 0.f;
 #pragma unroll
   for (int i = 0; i < 4; ++i)
@@ -216,18 +255,22 @@ template <bool Q8> __device__ __forceinline__ int vq_slot(int d) {
   }
 }
 
-template <int G, class T, bool Q8>
-__global__ __launch_bounds__(64) void k_attn_mx(AttnArgs a) {
-  constexpr int KW = kD / 2 + 4; // K row stride in words (padding spreads the banks)
-  constexpr int VW = kD + 16;    // V group stride in uint2
-  __shared__ __align__(16) uint32_t ks[kKeys][KW];
-  // (V[4j][d], V[4j+1][d]), (V[4j+2][d], V[4j+3][d]) at slot vq_slot(d)
-  __shared__ __align__(16) uint2 vq[kKeys / 4][VW];
-  const int split = blockIdx.x, kv = blockIdx.y, seq = attn_seq(a), lane = threadIdx.x;
+template <class T, bool Q8, int W>
+__global__ __launch_bounds__(64 * W) void k_attn_mx(AttnArgs a) {
+  constexpr int NB = 8 / W; // 16-dimension blocks of the output per wave
+  const int G = a.group;
+  // Per tile of the round: (V[4j][d], V[4j+1][d]), (V[4j+2][d], V[4j+3][d]) at slot
+  // vq_slot(d) ^ 16 (j % 2) (odd groups half the banks away from even ones); the probabilities in the A operand's layout; per query row, the tile's
+  // maximum, its rescale factor and its sum of probabilities.
+  __shared__ __align__(16) uint2 vq[W][kKeys / 4][kD];
+  __shared__ __align__(16) uint4 pq[W][64];
+  __shared__ __align__(16) float tile_max[W][16], tile_alpha[W][16], tile_total[W][16];
+  const int split = blockIdx.x, kv = blockIdx.y, lane = threadIdx.x & 63;
+  const int wave = W == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int col = lane & 15, grp = lane >> 4;
-  int n, first;
-  if (!attn_window(a, seq, n, first)) {
-    if (split == 0 && kv == 0 && lane == 0)
+  int seq, n, first;
+  if (!attn_pick(a, seq, n, first)) {
+    if (split == 0 && kv == 0 && threadIdx.x == 0)
       raise_bad(a.bad);
     return;
   }
@@ -236,22 +279,66 @@ __global__ __launch_bounds__(64) void k_attn_mx(AttnArgs a) {
     return; // block-uniform
   const int begin = tiles * split / active, end = tiles * (split + 1) / active;
   const int features = a.hkv * kD;
-  const size_t head_off = (size_t)seq * a.seq_stride * features + kv * kD;
-  const uint16_t *kc = a.kc + head_off, *vc = a.vc + head_off;
-  const int8_t *k8 = reinterpret_cast<const int8_t *>(a.kc) + head_off;
-  const int8_t *v8 = reinterpret_cast<const int8_t *>(a.vc) + head_off;
-  const float2 *sc = reinterpret_cast<const float2 *>(a.kvscales) +
-                     (size_t)seq * a.seq_stride * a.hkv + kv;
+  constexpr int ES = Q8 ? 1 : 2; // bytes per cache element
+  const size_t head_off = ((size_t)seq * a.seq_stride * features + kv * kD) * ES;
+  const char *kbytes = reinterpret_cast<const char *>(a.kc) + head_off;
+  const char *vbytes = reinterpret_cast<const char *>(a.vc) + head_off;
+  const char *sbytes = reinterpret_cast<const char *>(
+      reinterpret_cast<const float2 *>(a.kvscales) + (size_t)seq * a.seq_stride * a.hkv + kv);
 
-  // Query operand: row col (zero past G), dimensions 32 t + 8 grp + e; finite and
-  // BF16-exact, as the reference requires of its fp32 input.
+  // Tile loads, each instruction covering whole rows of the head (BF16: 256 B on 16 lanes;
+  // q8: 128 codes on 8 lanes): K straight into the score MFMAs' operand layout, 64 B of 16
+  // rows an instruction, reads at half the rate (128 workgroups: 3.3 TB/s against 6.1).
+  //  K: load m is key lane / KL + 64 / KL m, 16 bytes at chunk lane % KL of the row.
+  //  V: BF16 m = 4 h + p is key 16 h + 4 grp + p, dimensions 8 col ..; q8 m is key
+  //  4 (lane / 8) + m, dimensions 16 (lane % 8) ...
+  // Window offsets past the last key read the last key's row (the reference zero-fills
+  // them; their scores are masked to -inf, so their probabilities are 0).
+  constexpr int KL = Q8 ? 8 : 16, CH = Q8 ? 4 : 8;
+  uint4 kw[CH], vw[CH];
+  float ksc[2], vsc[4]; // q8: scales of keys 16 h + col (K) and of this lane's V keys
+  const uint32_t part = 16 * (lane & (KL - 1)), first_row = (uint32_t)(first % a.cap);
+  auto row_of = [&](int tile, int key) { // the window holds at most cap keys: one wrap
+    const uint32_t r = first_row + (uint32_t)min(tile * kKeys + key, n - 1);
+    return min(r, r - (uint32_t)a.cap); // r - cap is huge when r < cap
+  };
+  const uint32_t row_bytes = (uint32_t)features * ES, scale_bytes = (uint32_t)a.hkv * 8;
+  auto load_k = [&](int tile) {
+#pragma unroll
+    for (int m = 0; m < CH; ++m)
+      kw[m] = ld_nt(reinterpret_cast<const uint4 *>(
+          kbytes + part + (size_t)row_of(tile, lane / KL + 64 / KL * m) * row_bytes));
+    if constexpr (Q8) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+        ksc[h] = *reinterpret_cast<const float *>(sbytes + (size_t)row_of(tile, 16 * h + col) * scale_bytes);
+    }
+  };
+  auto load_v = [&](int tile) {
+#pragma unroll
+    for (int m = 0; m < CH; ++m) {
+      const uint32_t r = row_of(tile, 4 * (lane / KL) + (Q8 ? m : 16 * (m >> 2) + (m & 3)));
+      vw[m] = ld_nt(reinterpret_cast<const uint4 *>(vbytes + part + (size_t)r * row_bytes));
+      if constexpr (Q8)
+        vsc[m] = *reinterpret_cast<const float *>(sbytes + 4 + (size_t)r * scale_bytes);
+    }
+  };
+  if (begin + wave < end) { // wave-uniform
+    load_k(begin + wave);
+    load_v(begin + wave);
+  }
+  issue_point();
+
+  // Query operand: row col (zero past G), step t's dimensions as K's chunks hold them;
+  // finite and BF16-exact, as the reference requires of its fp32 input.
   uint4 qb[4];
   bool fine = true;
 #pragma unroll
   for (int t = 0; t < 4; ++t) {
     uint32_t w[4] = {0, 0, 0, 0};
     if (col < G) {
-      const size_t o = ((size_t)seq * a.hq + kv * G + col) * kD + 32 * t + 8 * grp;
+      const size_t o = ((size_t)seq * a.hq + kv * G + col) * kD +
+                       (Q8 ? 64 * (t >> 1) + 16 * grp + 8 * (t & 1) : 32 * t + 8 * grp);
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const float x0 = act_value<T>(a.q, o + 2 * e), x1 = act_value<T>(a.q, o + 2 * e + 1);
@@ -262,249 +349,230 @@ __global__ __launch_bounds__(64) void k_attn_mx(AttnArgs a) {
     }
     qb[t] = make_uint4(w[0], w[1], w[2], w[3]);
   }
-  if (__ballot(!fine) != 0 && lane == 0)
-    raise_bad(a.bad);
-  fine = true;
 
-  // Tile loads, each instruction covering whole rows of the head (BF16: 256 B on 16 lanes;
-  // q8: 128 codes on 8 lanes).
-  //  BF16 K: chunk c = lane + 64 m is key c / 16, dimensions 8 (c % 16) ..; V: m = 4 h + p
-  //  is key 16 h + 4 grp + p, dimensions 8 col ...
-  //  q8 K: chunk c = lane + 64 m is key c / 8, dimensions 16 (c % 8) ..; V: m = p is key
-  //  4 (lane / 8) + p, dimensions 16 (lane % 8) ..; each with its key's scale.
-  // Rows past the window load a valid row and are zeroed (the reference zero-fills them).
-  constexpr int CH = Q8 ? 4 : 8;
-  float ksc[CH], vsc[CH];
-  // Cache row of window offset tile * 32 + key: the tile's first row (one modulo per tile)
-  // plus the key, wrapped once (the window holds at most cap keys); keys past the window
-  // read the window's first row.
-  const int first_row = first % a.cap;
-  auto row_of = [&](int tile, int key) {
-    const int base = (first + tile * kKeys) % a.cap, r = base + key;
-    return (size_t)(tile * kKeys + key < n ? (r >= a.cap ? r - a.cap : r) : first_row);
-  };
-  auto vkey = [&](int m) {
-    return Q8 ? 4 * (lane >> 3) + m : 16 * (m >> 2) + 4 * grp + (m & 3);
-  };
-  // A tile whose 32 keys are inside the window and do not wrap is 32 consecutive cache
-  // rows from `base`: load m of a lane is then the tile's first row, plus this lane's
-  // offset for m = 0 (bytes), plus a per-m step that is the same for every lane.
-  //  q8 K: key lane / 8 + 8 m; V: key 4 (lane / 8) + m.  BF16 K: key lane / 16 + 4 m;
-  //  V: key 4 grp + 16 (m / 4) + m % 4.
-  constexpr int ES = Q8 ? 1 : 2; // bytes per cache element
-  const size_t row_bytes = (size_t)features * ES;
-  const uint32_t koff = (uint32_t)(Q8 ? (lane >> 3) * row_bytes + 16 * (lane & 7)
-                                      : (lane >> 4) * row_bytes + 16 * (lane & 15));
-  const uint32_t voff = (uint32_t)(Q8 ? 4 * (lane >> 3) * row_bytes + 16 * (lane & 7)
-                                      : 4 * grp * row_bytes + 16 * col);
-  const uint32_t kso = (uint32_t)((lane >> 3) * a.hkv * 8), vso = 4 * kso + 4;
-  auto kstep = [&](int m) { return (size_t)(Q8 ? 8 * m : 4 * m) * row_bytes; };
-  auto vstep = [&](int m) { return (size_t)(Q8 ? m : 16 * (m >> 2) + (m & 3)) * row_bytes; };
-  const char *kbytes = Q8 ? reinterpret_cast<const char *>(k8) : reinterpret_cast<const char *>(kc);
-  const char *vbytes = Q8 ? reinterpret_cast<const char *>(v8) : reinterpret_cast<const char *>(vc);
-  const char *sbytes = reinterpret_cast<const char *>(sc);
-  auto load_tile = [&](int tile, uint4 (&kw)[8], uint4 (&vw)[8]) {
-    const int base = (first + tile * kKeys) % a.cap;
-    if (tile * kKeys + kKeys <= n && base + kKeys <= a.cap) { // block-uniform
-      const char *kt = kbytes + (size_t)base * row_bytes, *vt = vbytes + (size_t)base * row_bytes;
-      const char *st = sbytes + (size_t)base * a.hkv * 8;
+  float maximum = -INFINITY, den = 0.f; // of row col, over the tiles before this round
+  f32x4_t o[NB];
 #pragma unroll
-      for (int m = 0; m < CH; ++m) {
-        kw[m] = ld_nt(reinterpret_cast<const uint4 *>(kt + kstep(m) + koff));
-        vw[m] = ld_nt(reinterpret_cast<const uint4 *>(vt + vstep(m) + voff));
-        if constexpr (Q8) {
-          ksc[m] = *reinterpret_cast<const float *>(st + (size_t)8 * m * a.hkv * 8 + kso);
-          vsc[m] = *reinterpret_cast<const float *>(st + (size_t)m * a.hkv * 8 + vso);
-        }
-      }
-      return;
-    }
-#pragma unroll
-    for (int m = 0; m < CH; ++m) {
-      const int c = lane + 64 * m;
-      const size_t kr = row_of(tile, c >> (Q8 ? 3 : 4)), vr = row_of(tile, vkey(m));
-      if constexpr (Q8) {
-        kw[m] = ld_nt(reinterpret_cast<const uint4 *>(k8 + kr * features) + (c & 7));
-        vw[m] = ld_nt(reinterpret_cast<const uint4 *>(v8 + vr * features) + (lane & 7));
-        ksc[m] = sc[kr * a.hkv].x;
-        vsc[m] = sc[vr * a.hkv].y;
-      } else {
-        kw[m] = ld_nt(reinterpret_cast<const uint4 *>(kc + kr * features) + (c & 15));
-        vw[m] = ld_nt(reinterpret_cast<const uint4 *>(vc + vr * features) + col);
-      }
-    }
-  };
-
-  float maximum = -INFINITY, den = 0.f;
-  f32x4_t o[8];
-#pragma unroll
-  for (int b = 0; b < 8; ++b)
+  for (int b = 0; b < NB; ++b)
     o[b] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  uint4 kw[8], vw[8];
-  load_tile(begin, kw, vw);
-  for (int tile = begin; tile < end; ++tile) {
-    const int left = n - tile * kKeys; // keys of this tile inside the window (may be >= 32)
-    // Stage K rows and V key groups as BF16.
-    if constexpr (Q8) {
-      if (left < kKeys) { // block-uniform: the window's last tile
-#pragma unroll
-        for (int m = 0; m < CH; ++m) {
-          if (((lane + 64 * m) >> 3) >= left) {
-            kw[m] = make_uint4(0, 0, 0, 0);
-            ksc[m] = 1.f;
-          }
-        }
+  for (int round = begin; round < end; round += W) {
+    const int count = min(W, end - round), tile = round + wave;
+    float sv[8], tmax = -INFINITY;
+    // A wave's tile up to its maximum score.  MORE: the wave has a tile in the next round,
+    // loaded as soon as the registers are free (K once it is in LDS, V likewise).  The last
+    // tile is code of its own: with the loads under a condition the compiler can only wait
+    // for all of them at once, which exposed the latency of the tile just issued
+    // (W = 1: 148 -> 211 us at 131072 keys).
+    auto scores = [&](auto more) {
+      constexpr bool MORE = decltype(more)::value;
+      const int left = n - tile * kKeys; // keys of this tile inside the window (may be >= 32)
+      // Scores: lane holds row col, keys 16 h + 4 grp + i.
+      f32x4_t s[2] = {f32x4_t{0.f, 0.f, 0.f, 0.f}, f32x4_t{0.f, 0.f, 0.f, 0.f}};
+      // The tile's K rows cross the wave's LDS image (chunks exchanged by key, so that no two
+      // lanes of a 16-lane group meet in a bank), then its V rows take the same space: one
+      // wave's LDS accesses run in program order, so the K reads come first.
+      uint4 *kq = reinterpret_cast<uint4 *>(&vq[wave][0][0]);
+      if constexpr (Q8) {
 #pragma unroll
         for (int m = 0; m < 4; ++m) {
-          if (vkey(m) >= left) {
-            vw[m] = make_uint4(0, 0, 0, 0);
-            vsc[m] = 1.f;
+          const int key = lane / 8 + 8 * m;
+          kq[8 * key + ((lane & 7) ^ ((key >> 1) & 7))] = kw[m];
+        }
+        const float kscale[2] = {ksc[0], ksc[1]};
+        if constexpr (MORE) {
+          load_k(tile + W);
+          issue_point();
+        }
+        // Decoded a chunk at a time: the scheduling barriers keep one chunk's values in
+        // registers, not all of them (256 VGPRs and spills without).
+        float least = 0.f;
+        // Whether some key's scale needs every value checked (rare: huge or invalid scales).
+        const bool kslow = __ballot(!q8_scale_fast(kscale[0]) || !q8_scale_fast(kscale[1])) != 0;
+        const bool vslow = __ballot(!q8_scale_fast(vsc[0]) || !q8_scale_fast(vsc[1]) ||
+                                    !q8_scale_fast(vsc[2]) || !q8_scale_fast(vsc[3])) != 0;
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+          for (int u = 0; u < 2; ++u) {
+            const uint4 c = kq[8 * (16 * h + col) + ((4 * u + grp) ^ (col >> 1))];
+            uint32_t w[8];
+            float f[8];
+            q8_values8(c.x, c.y, kscale[h], f, least);
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+              w[e] = pack2(f[2 * e], f[2 * e + 1]);
+            q8_values8(c.z, c.w, kscale[h], f, least);
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+              w[4 + e] = pack2(f[2 * e], f[2 * e + 1]);
+            s[h] = mfma_bf16(make_uint4(w[0], w[1], w[2], w[3]), qb[2 * u], s[h]);
+            s[h] = mfma_bf16(make_uint4(w[4], w[5], w[6], w[7]), qb[2 * u + 1], s[h]);
+            if constexpr (W > 1)
+              __builtin_amdgcn_sched_barrier(0);
           }
+        if (kslow) { // one rare branch, not one per chunk, which would cut the code above apart
+#pragma unroll
+          for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int u = 0; u < 2; ++u)
+              if (!q8_scale_fast(kscale[h]))
+                fine = fine && q8_check16(kq[8 * (16 * h + col) + ((4 * u + grp) ^ (col >> 1))],
+                                          kscale[h]);
         }
-      }
-      float least = 0.f;
-      bool slow = false;
+        const int t7 = lane & 7, j = lane >> 3;
+        uint2 *dst = &vq[wave][j][(16 * t7) ^ ((j & 1) << 4)];
 #pragma unroll
-      for (int m = 0; m < CH; ++m) {
-        const int c = lane + 64 * m, key = c >> 3, part = c & 7;
-        float f[16];
-        q8_values16(kw[m], ksc[m], f, least, slow);
-        uint32_t w[8];
+        for (int i = 0; i < 4; ++i) { // dimensions 4 i .. 4 i + 3 of the chunk, four keys
+          float f[4][4];
 #pragma unroll
-        for (int e = 0; e < 8; ++e)
-          w[e] = pack2(f[2 * e], f[2 * e + 1]);
-        *reinterpret_cast<uint4 *>(&ks[key][part * 8]) = make_uint4(w[0], w[1], w[2], w[3]);
-        *reinterpret_cast<uint4 *>(&ks[key][part * 8 + 4]) = make_uint4(w[4], w[5], w[6], w[7]);
-      }
-      float fv[4][16];
+          for (int m = 0; m < 4; ++m)
+            q8_values4(i == 0 ? vw[m].x : i == 1 ? vw[m].y : i == 2 ? vw[m].z : vw[m].w, vsc[m],
+                       f[m], least);
 #pragma unroll
-      for (int m = 0; m < 4; ++m)
-        q8_values16(vw[m], vsc[m], fv[m], least, slow);
-      fine = fine && least > -128.f;
-      if (__ballot(slow) != 0) { // rare: huge or invalid scales
-#pragma unroll
-        for (int m = 0; m < CH; ++m) {
-          if (((lane + 64 * m) >> 3) < left && !q8_scale_fast(ksc[m]))
-            fine = fine && q8_check16(kw[m], ksc[m]);
-          if (vkey(m) < left && !q8_scale_fast(vsc[m]))
-            fine = fine && q8_check16(vw[m], vsc[m]);
+          for (int e = 0; e < 4; e += 2)
+            *reinterpret_cast<uint4 *>(dst + 2 * ((2 * i + e / 2 + t7) & 7)) =
+                make_uint4(pack2(f[0][e], f[1][e]), pack2(f[2][e], f[3][e]),
+                           pack2(f[0][e + 1], f[1][e + 1]), pack2(f[2][e + 1], f[3][e + 1]));
+          if constexpr (W > 1)
+            __builtin_amdgcn_sched_barrier(0);
         }
-      }
-      const int t7 = lane & 7;
-      uint2 *dst = &vq[lane >> 3][16 * t7];
+        fine = fine && least > -128.f;
+        if (vslow) {
 #pragma unroll
-      for (int e = 0; e < 16; e += 2)
-        *reinterpret_cast<uint4 *>(dst + 2 * ((e / 2 + t7) & 7)) =
-            make_uint4(pack2(fv[0][e], fv[1][e]), pack2(fv[2][e], fv[3][e]),
-                       pack2(fv[0][e + 1], fv[1][e + 1]), pack2(fv[2][e + 1], fv[3][e + 1]));
-    } else {
-      if (left < kKeys) { // block-uniform: the window's last tile
+          for (int m = 0; m < 4; ++m)
+            if (!q8_scale_fast(vsc[m]))
+              fine = fine && q8_check16(vw[m], vsc[m]);
+        }
+      } else {
 #pragma unroll
         for (int m = 0; m < 8; ++m) {
-          if (((lane + 64 * m) >> 4) >= left)
-            kw[m] = make_uint4(0, 0, 0, 0);
-          if (vkey(m) >= left)
-            vw[m] = make_uint4(0, 0, 0, 0);
+          const int key = grp + 4 * m;
+          kq[16 * key + (col ^ (key & 15))] = kw[m];
+        }
+        if constexpr (MORE) {
+          load_k(tile + W);
+          issue_point();
+        }
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+          for (int t = 0; t < 4; ++t)
+            s[h] = mfma_bf16(kq[16 * (16 * h + col) + ((4 * t + grp) ^ col)], qb[t], s[h]);
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const uint4 *p = &vw[4 * h];
+          const uint32_t w0[4] = {p[0].x, p[0].y, p[0].z, p[0].w}, w1[4] = {p[1].x, p[1].y, p[1].z, p[1].w},
+                         w2[4] = {p[2].x, p[2].y, p[2].z, p[2].w}, w3[4] = {p[3].x, p[3].y, p[3].z, p[3].w};
+          uint2 *dst = &vq[wave][4 * h + grp][(8 * col) ^ ((grp & 1) << 4)];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) // dimensions 2e, 2e + 1 of the chunk
+            *reinterpret_cast<uint4 *>(dst + 2 * ((e + (col >> 2)) & 3)) = make_uint4(
+                __builtin_amdgcn_perm(w1[e], w0[e], 0x05040100u),
+                __builtin_amdgcn_perm(w3[e], w2[e], 0x05040100u),
+                __builtin_amdgcn_perm(w1[e], w0[e], 0x07060302u),
+                __builtin_amdgcn_perm(w3[e], w2[e], 0x07060302u));
         }
       }
-#pragma unroll
-      for (int m = 0; m < 8; ++m) {
-        const int c = lane + 64 * m;
-        *reinterpret_cast<uint4 *>(&ks[c >> 4][(c & 15) * 4]) = kw[m];
+      if constexpr (MORE) {
+        load_v(tile + W);
+        issue_point();
       }
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const uint4 *p = &vw[4 * h];
-        const uint32_t w0[4] = {p[0].x, p[0].y, p[0].z, p[0].w}, w1[4] = {p[1].x, p[1].y, p[1].z, p[1].w},
-                       w2[4] = {p[2].x, p[2].y, p[2].z, p[2].w}, w3[4] = {p[3].x, p[3].y, p[3].z, p[3].w};
-        uint2 *dst = &vq[4 * h + grp][8 * col];
+      for (int h = 0; h < 2; ++h)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) // dimensions 2e, 2e + 1 of the chunk
-          *reinterpret_cast<uint4 *>(dst + 2 * ((e + (col >> 2)) & 3)) = make_uint4(
-              __builtin_amdgcn_perm(w1[e], w0[e], 0x05040100u),
-              __builtin_amdgcn_perm(w3[e], w2[e], 0x05040100u),
-              __builtin_amdgcn_perm(w1[e], w0[e], 0x07060302u),
-              __builtin_amdgcn_perm(w3[e], w2[e], 0x07060302u));
+        for (int i = 0; i < 4; ++i) {
+          float v = s[h][i] * kScoreScale;
+          if (16 * h + 4 * grp + i < left)
+            fine = fine && isfinite(v);
+          else
+            v = -INFINITY;
+          sv[4 * h + i] = v;
+          tmax = fmaxf(tmax, v);
+        }
+      tmax = fmaxf(tmax, lane_xor<16>(tmax));
+      tmax = fmaxf(tmax, lane_xor<32>(tmax));
+    };
+    if (tile + W < end) // wave-uniform
+      scores(std::true_type{});
+    else if (tile < end)
+      scores(std::false_type{});
+    if (W > 1 && grp == 0)
+      tile_max[wave][col] = tmax; // -inf without a tile
+    // The running maximum at this wave's tile (every tile of the round before it counted),
+    // and after the round.
+    float before = maximum, after = fmaxf(maximum, tmax);
+    if constexpr (W > 1) {
+      __syncthreads();
+      after = maximum;
+#pragma unroll
+      for (int t = 0; t < W; ++t) {
+        const float m = tile_max[t][col];
+        before = fmaxf(before, t < wave ? m : -INFINITY);
+        after = fmaxf(after, m);
       }
     }
+    uint4 pa;
+    float alpha, total = 0.f;
+    if (wave < count) {
+      const float next = fmaxf(before, tmax);
+      alpha = isfinite(before) ? __expf(before - next) : 0.f;
+      float p[8];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        p[k] = isfinite(sv[k]) ? __expf(sv[k] - next) : 0.f;
+        total += p[k];
+      }
+      total += lane_xor<16>(total);
+      total += lane_xor<32>(total);
+      pa = make_uint4(pack2(p[0], p[1]), pack2(p[2], p[3]), pack2(p[4], p[5]), pack2(p[6], p[7]));
+      if constexpr (W > 1)
+        pq[wave][lane] = pa;
+      if (grp == 0) {
+        tile_alpha[wave][col] = alpha;
+        tile_total[wave][col] = total;
+      }
+    }
+    maximum = after;
     __syncthreads();
-    // The next tile's loads are in flight during this tile's arithmetic (the last tile
-    // reloads itself, keeping the loads unconditional).
-    load_tile(min(tile + 1, end - 1), kw, vw);
-
-    // Scores: lane holds row col, keys 16 h + 4 grp + i.
-    f32x4_t s[2];
+    // PV of this wave's output blocks over the round's tiles, in tile order.
+    auto pv = [&](int t) {
+      const uint4 pt = W > 1 ? pq[t][lane] : pa;
+      const float4 ar = *reinterpret_cast<const float4 *>(&tile_alpha[t][4 * grp]);
+      den = __builtin_fmaf(den, W > 1 ? tile_alpha[t][col] : alpha, W > 1 ? tile_total[t][col] : total);
+      const f32x4_t rescale = {ar.x, ar.y, ar.z, ar.w}; // 1 unless a row's maximum moved
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      s[h] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int t = 0; t < 4; ++t)
-        s[h] = mfma_bf16(*reinterpret_cast<const uint4 *>(&ks[16 * h + col][16 * t + 4 * grp]),
-                         qb[t], s[h]);
-    }
-    float sv[8], tmax = -INFINITY;
-#pragma unroll
-    for (int h = 0; h < 2; ++h)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        float v = s[h][i] * kScoreScale;
-        if (16 * h + 4 * grp + i < left)
-          fine = fine && isfinite(v);
-        else
-          v = -INFINITY;
-        sv[4 * h + i] = v;
-        tmax = fmaxf(tmax, v);
+      for (int b = 0; b < NB; ++b) {
+        const int d = vq_slot<Q8>(16 * (NB * wave + b) + col) ^ ((grp & 1) << 4);
+        const uint2 v0 = vq[t][grp][d], v1 = vq[t][4 + grp][d];
+        o[b] = mfma_bf16(pt, make_uint4(v0.x, v0.y, v1.x, v1.y), o[b] * rescale);
       }
-    tmax = fmaxf(tmax, lane_xor<16>(tmax));
-    tmax = fmaxf(tmax, lane_xor<32>(tmax));
-    const float next = fmaxf(maximum, tmax);
-    const float alpha = isfinite(maximum) ? __expf(maximum - next) : 0.f;
-    float p[8], total = 0.f;
+    };
+    if (count == W) { // block-uniform; without a test per tile its LDS reads overlap
 #pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      p[k] = isfinite(sv[k]) ? __expf(sv[k] - next) : 0.f;
-      total += p[k];
-    }
-    total += lane_xor<16>(total);
-    total += lane_xor<32>(total);
-    den = __builtin_fmaf(den, alpha, total);
-    maximum = next;
-    const uint4 pa = make_uint4(pack2(p[0], p[1]), pack2(p[2], p[3]), pack2(p[4], p[5]),
-                                pack2(p[6], p[7]));
-    if (__ballot(alpha != 1.f) != 0) { // wave-uniform
-      float ar[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        ar[i] = __shfl(alpha, 4 * grp + i, 64);
-#pragma unroll
-      for (int b = 0; b < 8; ++b)
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          o[b][i] *= ar[i];
-    }
-#pragma unroll
-    for (int b = 0; b < 8; ++b) {
-      const int d = vq_slot<Q8>(16 * b + col);
-      const uint2 v0 = vq[grp][d], v1 = vq[4 + grp][d];
-      o[b] = mfma_bf16(pa, make_uint4(v0.x, v0.y, v1.x, v1.y), o[b]);
+      for (int t = 0; t < W; ++t)
+        pv(t);
+    } else {
+      for (int t = 0; t < count; ++t)
+        pv(t);
     }
     __syncthreads();
   }
-  // Rows 4 grp + i: this lane's dimension 16 b + col of each.
+  // Rows 4 grp + i: this lane's dimension 16 (NB wave + b) + col of each.
   const int head0 = kv * G;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int r = 4 * grp + i;
     const float d = __shfl(den, r, 64), mx = __shfl(maximum, r, 64);
     if (r < G) {
-      float *dst = a.partial + (((size_t)seq * a.splits + split) * a.hq + head0 + r) * kD + col;
+      float *dst = a.partial + (((size_t)seq * a.splits + split) * a.hq + head0 + r) * kD +
+                   16 * NB * wave + col;
 #pragma unroll
-      for (int b = 0; b < 8; ++b) {
+      for (int b = 0; b < NB; ++b) {
         const float v = o[b][i] / d;
         fine = fine && isfinite(v);
         dst[16 * b] = v;
       }
-      if (col == 0) {
+      if (col == 0 && wave == 0) {
         const float l = mx + logf(d);
         fine = fine && isfinite(l);
         a.lse[((size_t)seq * a.splits + split) * a.hq + head0 + r] = l;
@@ -750,15 +818,15 @@ template <int G> __global__ __launch_bounds__(256) void k_q8_0_mx(AttnArgs a) {
   __shared__ float ksc_all[4][32][4];    // K block scales by key
   __shared__ float vsc_all[4][4][32];    // V block scales by block
   __shared__ float ps_all[4][8][36];     // probabilities by head (rows padded)
-  const int split = blockIdx.x, seq = attn_seq(a), tid = threadIdx.x, kv = tid >> 6;
+  const int split = blockIdx.x, tid = threadIdx.x, kv = tid >> 6;
   const int lane = tid & 63, col = lane & 15, grp = lane >> 4;
   auto &kq = kq_all[kv].r;
   auto &vq = vq_all[kv].r;
   auto &ksc = ksc_all[kv];
   auto &vsc = vsc_all[kv];
   auto &ps = ps_all[kv];
-  int n, first;
-  if (!attn_window(a, seq, n, first) || (a.local && a.cap != 1024)) {
+  int seq, n, first;
+  if (!attn_pick(a, seq, n, first) || (a.local && a.cap != 1024)) {
     if (split == 0 && tid == 0)
       raise_bad(a.bad);
     return;
@@ -1210,12 +1278,14 @@ int decode_attention(void *stream, const void *q, const padra_KVCache *kv, void 
   // Longest windows first when the lengths can differ much: several sequences on a
   // global cache (a local ring's windows are at most 1024 keys).
   const long long obase = qbase + (q8 ? (long long)seqs * q_heads * (kD / 4 + 4) : 0);
-  a.order = seqs >= 2 && seqs <= kOrderMaxSeqs && !local ? reinterpret_cast<int *>(scratch + obase)
-                                                         : nullptr;
+  const bool ordered = seqs >= 2 && seqs <= kOrderMaxSeqs && !local;
+  a.rank = ordered && seqs <= kRankMaxSeqs && !q8; // (q8_0's query kernel ranks them)
+  a.order = ordered && !a.rank ? reinterpret_cast<int *>(scratch + obase) : nullptr;
   a.decode = pos->decode;
   a.seqs = seqs;
   a.hq = q_heads;
   a.hkv = kv_heads;
+  a.group = q_heads / kv_heads;
   a.cap = kv->cap;
   a.local = local ? 1 : 0;
   a.splits = splits;
@@ -1252,27 +1322,34 @@ int decode_attention(void *stream, const void *q, const padra_KVCache *kv, void 
       hipLaunchKernelGGL((k_q8_0_mx_merge<T>), merge_grid, dim3(64), 0, s, a);
       return launched("DecodeAttention");
     }
-    auto split = [&](auto q8tag) {
+    auto split = [&](auto q8tag, auto wtag) {
       constexpr bool Q8 = decltype(q8tag)::value;
-      switch (group) {
-      case 1:
-        hipLaunchKernelGGL((k_attn_mx<1, T, Q8>), split_grid, dim3(64), 0, s, a);
-        break;
-      case 2:
-        hipLaunchKernelGGL((k_attn_mx<2, T, Q8>), split_grid, dim3(64), 0, s, a);
-        break;
-      case 4:
-        hipLaunchKernelGGL((k_attn_mx<4, T, Q8>), split_grid, dim3(64), 0, s, a);
-        break;
-      default:
-        hipLaunchKernelGGL((k_attn_mx<8, T, Q8>), split_grid, dim3(64), 0, s, a);
-        break;
-      }
+      constexpr int W = decltype(wtag)::value;
+      hipLaunchKernelGGL((k_attn_mx<T, Q8, W>), split_grid, dim3(64 * W), 0, s, a);
+    };
+    // Waves per workgroup, by how many workgroups the launch has: with few of them one wave
+    // each leaves most of the chip idle, with many the round's barriers cost more than its
+    // waves bring.  Measured (us, split and merge, W = 1 / 2 / 4 / 8; BF16, then q8):
+    //   1 sequence, 32768 keys, 32 heads (128 workgroups)  45.7/36.2/27.5/26.4  72.0/47.4/29.7/25.9
+    //   4 sequences, to 8000 keys, 32 heads (512)          21.9/19.3/17.9/21.8  27.7/21.3/17.2/21.5
+    //   8 sequences, the same (1024)                       27.2/25.3/27.8/36.4  29.1/24.9/25.9/36.8
+    //   16 sequences, 16 heads (2048)                      36.6/37.0/43.6/62.9  32.2/34.6/38.4/64.0
+    const int wgs = splits * kv_heads * seqs;
+    auto split_w = [&](auto q8tag) {
+      if (wgs <= 256)
+        split(q8tag, std::integral_constant<int, 8>{});
+      else if (wgs <= 512)
+        split(q8tag, std::integral_constant<int, 4>{});
+      else if (wgs <= 1024 && !local) // a local ring's split has two tiles or so: 15.2 us
+                                      // with two waves, 14.9 with one (12 sequences)
+        split(q8tag, std::integral_constant<int, 2>{});
+      else
+        split(q8tag, std::integral_constant<int, 1>{});
     };
     if (q8s)
-      split(std::true_type{});
+      split_w(std::true_type{});
     else
-      split(std::false_type{});
+      split_w(std::false_type{});
     if (fp8)
       hipLaunchKernelGGL((k_attn_merge_fp8<T>), dim3(seqs), dim3(256), 0, s, a, packed, scales);
     else

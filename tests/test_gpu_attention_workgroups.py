@@ -1,0 +1,105 @@
+"""Decode attention with one to eight waves per split (the launch's size picks the count): the
+same sequence gives the same bits in batches of every size, and the oracle's result alone."""
+import numpy as np
+import pytest
+import torch
+
+from padra_amd import abi, ops, synth
+
+from attn_tolerance import attn_close, bound_bf16
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module", autouse=True)
+def gpu():
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    abi.lib()
+    yield
+    torch.cuda.synchronize()
+
+
+def _rows(fmt, rng, rows):
+    """A cache plane as stored: BF16 bits, or codes."""
+    if fmt == abi.KV_BF16:
+        return synth.bf16_bits(rng.standard_normal((rows, 512)).astype(np.float32)).view(np.int16)
+    return rng.integers(-127, 128, (rows, 512)).astype(np.int8)
+
+
+@pytest.mark.parametrize("fmt", [abi.KV_BF16, abi.KV_Q8])
+@pytest.mark.parametrize("local", [False, True])
+def test_decode_attention_workgroup_sizes(oracle, fmt, local):
+    """17 sequences of 1 to 4096 keys (tile and round edges; local rings that wrap inside a
+    tile), run in batches of 17 (one wave a split), 8 (two), 3 (four) and 1 (eight); 32 query
+    heads on 4 KV heads, 32 splits (local: 16, so batches of 17, 12, 6 and 1: one, one, four, eight)."""
+    hq, hkv, capacity = 32, 4, 4096
+    cap = 1024 if local else capacity
+    windows = [1, 31, 32, 33, 64, 255, 256, 257, 1023, 1024, 1025, 1500, 2047, 2049, 4000, 4095,
+               4096]
+    seqs = len(windows)
+    batches = (17, 12, 6, 1) if local else (17, 8, 3, 1)
+    print(f"[case] attention workgroups fmt={fmt} local={local}", flush=True)
+    rng = np.random.default_rng(31 + fmt + 2 * local)
+    q = synth.bf16_bits((rng.standard_normal((seqs, hq, 128)) * 2).astype(np.float32))
+    kc, vc = _rows(fmt, rng, seqs * cap), _rows(fmt, rng, seqs * cap)
+    sc = rng.uniform(.005, .02, (seqs * cap, hkv, 2)).astype(np.float32)
+    states = np.array([[5, n - 1, capacity, 10, n - 1, min(n - 1, 1024), 0, 0] for n in windows],
+                      np.int32)
+    kd, vd, sd = (torch.from_numpy(a).cuda() for a in (kc, vc, sc))
+    qd = torch.from_numpy(q.view(np.int16)).cuda()
+    bad = torch.zeros(1, dtype=torch.int32, device="cuda")
+    outs = []
+    for size in batches:
+        out = torch.empty((seqs, hq, 128), dtype=torch.int16, device="cuda")
+        for at in range(0, seqs, size):
+            some = slice(at, min(seqs, at + size))
+            rows = slice(at * cap, some.stop * cap)
+            kv = ops.kv_cache(fmt, kd[rows], vd[rows], cap,
+                              scales=sd[rows] if fmt == abi.KV_Q8 else None, seq_stride=cap)
+            ops.DecodeAttention(qd[some], kv, out[some],
+                                ops.positions_decode(torch.from_numpy(states[some]).cuda(),
+                                                     maximum=capacity), bad, kv_heads=hkv,
+                                local=local)
+        torch.cuda.synchronize()
+        outs.append(out.cpu().numpy().view(np.uint16))
+    assert bad.item() == 0
+    for got in outs[1:]:
+        assert np.array_equal(got, outs[0])
+    for s in (0, 3, 7, 10, 16):
+        k, v = kc[s * cap:(s + 1) * cap], vc[s * cap:(s + 1) * cap]
+        if fmt == abi.KV_BF16:
+            k, v = k.view(np.uint16), v.view(np.uint16)
+        else:
+            scale = sc[s * cap:(s + 1) * cap]
+            k, v = (synth.bf16_bits(c.reshape(cap, hkv, 128).astype(np.float32) *
+                                    scale[..., i:i + 1]).reshape(cap, -1)
+                    for i, c in enumerate((k, v)))
+        want, used, wbad = oracle.decode_attention(q[s], k, v, windows[s] - 1, local=local)
+        assert not wbad
+        close, d = attn_close(outs[0][s], want,
+                              bound_bf16(q[s], k, v, windows[s] - 1, local, used))
+        assert close.all(), (windows[s], int(d.max()))
+
+
+def test_decode_attention_rows_past_4gib():
+    """A cache of 131072 rows of 160 KV heads (5.4 GB a plane): row offsets past 2^32 bytes.
+    Heads taken out into a cache of four give the same bits."""
+    hkv, cap, n = 160, 131072, 131072
+    print("[case] attention rows past 4 GiB", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(5)
+    kc, vc = (torch.randn((cap, hkv * 128), generator=g, device="cuda", dtype=torch.bfloat16)
+              for _ in range(2))
+    q = torch.randn((1, hkv, 128), generator=g, device="cuda").bfloat16()
+    states = torch.tensor([[5, n - 1, cap, 10, n - 1, 1024, 0, 0]], dtype=torch.int32, device="cuda")
+    bad = torch.zeros(1, dtype=torch.int32, device="cuda")
+    pos = ops.positions_decode(states, maximum=cap)
+    out = torch.empty_like(q)
+    ops.DecodeAttention(q, ops.kv_cache(abi.KV_BF16, kc, vc, cap), out, pos, bad, kv_heads=hkv)
+    for h in (0, 124, 156):
+        k4, v4 = (t[:, h * 128:(h + 4) * 128].contiguous() for t in (kc, vc))
+        some, q4 = torch.empty((1, 4, 128), dtype=torch.bfloat16, device="cuda"), q[:, h:h + 4].contiguous()
+        ops.DecodeAttention(q4, ops.kv_cache(abi.KV_BF16, k4, v4, cap), some, pos, bad, kv_heads=4)
+        torch.cuda.synchronize()
+        assert torch.equal(some, out[:, h:h + 4])
+    assert bad.item() == 0
