@@ -583,30 +583,61 @@ __global__ __launch_bounds__(64 * W) void k_attn_mx(AttnArgs a) {
     raise_bad(a.bad);
 }
 
+// Partial outputs of one (sequence, head), a float2 per lane and split.  The merge kernels are
+// bound by their chain of memory round trips (control record, log-sum-exps, partials), so they issue every split's load before the first use and, in small launches,
+// before the control record is there: the splits that turn out inactive are read in vain,
+// inside the scratch.  Launches of more heads read only the active ones: there the bytes count.
+// Steps of 1 / 8 / 64 sequences (1000, 8000, 8000 keys), before -> after: BF16 10.3 -> 8.5,
+// 25.2 -> 23.8, 103.6 -> 104.2 us; q8_0 21.9 -> 20.3, 39.2 -> 31.6, 107.1 -> 102.6 us.
+constexpr int kMaxSplits = 32, kEarlyHeads = 512;
+
+__device__ __forceinline__ void merge_load(const float *src, size_t step, int count,
+                                           float2 (&p)[kMaxSplits]) {
+#pragma unroll
+  for (int g = 0; g < kMaxSplits; g += 4)
+    if (g < count) { // wave-uniform
+#pragma unroll
+      for (int i = g; i < g + 4; ++i)
+        p[i] = *reinterpret_cast<const float2 *>(src + min(i, count - 1) * step);
+    }
+}
+
+// The weighted sum in split order: w holds split sp's weight in lane sp.
+__device__ __forceinline__ void merge_sum(const float2 (&p)[kMaxSplits], float w, int active,
+                                          float &s0, float &s1) {
+  s0 = s1 = 0.f;
+#pragma unroll
+  for (int sp = 0; sp < kMaxSplits; ++sp)
+    if (sp < active) {
+      const float ws =
+          __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), sp));
+      s0 = __builtin_fmaf(ws, p[sp].x, s0);
+      s1 = __builtin_fmaf(ws, p[sp].y, s1);
+    }
+}
+
 template <class T> __global__ __launch_bounds__(64) void k_attn_merge(AttnArgs a) {
-  __shared__ float weights[32];
   const int head = blockIdx.x, seq = blockIdx.y, lane = threadIdx.x;
+  const size_t entry = (size_t)seq * a.splits * a.hq + head, step = (size_t)a.hq * kD;
+  const float *src = a.partial + entry * kD + 2 * lane;
+  const bool early = gridDim.x * gridDim.y <= kEarlyHeads;
+  const float lse = a.lse[entry + (size_t)min(lane, a.splits - 1) * a.hq];
+  float2 p[kMaxSplits];
+  if (early)
+    merge_load(src, step, a.splits, p);
   int n, first;
   if (!attn_window(a, seq, n, first))
     return; // the split kernel raised the flag
   const int active = min(a.splits, (n + kKeys - 1) / kKeys);
-  const float v = lane < active ? a.lse[((size_t)seq * a.splits + lane) * a.hq + head] : -INFINITY;
+  if (!early)
+    merge_load(src, step, active, p);
+  const float v = lane < active ? lse : -INFINITY;
   const float mx = xor_max32(v);
   const float w = lane < active ? expf(v - mx) : 0.f;
-  const float total = xor_sum32(w);
-  bool fine = true;
-  if (lane < active) {
-    weights[lane] = w / total;
-    fine = isfinite(weights[lane]);
-  }
-  __syncthreads();
-  float s0 = 0.f, s1 = 0.f;
-  for (int sp = 0; sp < active; ++sp) {
-    const float2 p = *reinterpret_cast<const float2 *>(
-        a.partial + (((size_t)seq * a.splits + sp) * a.hq + head) * kD + 2 * lane);
-    s0 = __builtin_fmaf(weights[sp], p.x, s0);
-    s1 = __builtin_fmaf(weights[sp], p.y, s1);
-  }
+  const float total = xor_sum32(w), weight = w / total;
+  bool fine = lane >= active || isfinite(weight);
+  float s0, s1;
+  merge_sum(p, weight, active, s0, s1);
   const uint32_t word = pack2(s0, s1);
   fine = fine && ((word & 0x7f80u) != 0x7f80u) && ((word & 0x7f800000u) != 0x7f800000u);
   const size_t o = ((size_t)seq * a.hq + head) * kD + 2 * lane;
@@ -619,70 +650,49 @@ template <class T> __global__ __launch_bounds__(64) void k_attn_merge(AttnArgs a
     raise_bad(a.bad);
 }
 
-
 // MergeQuantize (attention_merge_quantize_wide_exact.cuh:9-66), the merge the reference
 // runs after its q8 split (attention_gqa8_q8.cuh:278-300) and, with the FP8 output, after
-// the BF16 one: the per-head merge of k_attn_merge for every head of a sequence in one
-// workgroup, then the E4M3 encoding of the whole output row (q_heads x 128 values) with
-// scale = max|out| / 448 (1 for a zero row), as padra_QuantizeFP8 writes it.  Waves take
-// heads wave, wave + 4, ...; lane l holds dimensions 2l, 2l + 1 of each.
+// the BF16 one: k_attn_merge, then this kernel, the E4M3 encoding of each sequence's output
+// row (q_heads x 128 values) with scale = max|out| / 448 (1 for a zero row), as
+// padra_QuantizeFP8 writes it.  Waves take heads wave, wave + 4, ...; lane l holds
+// dimensions 2l, 2l + 1 of each.  The row's maximum needs every head, and one workgroup that
+// merges 32 heads of 32 splits (512 KB) for it runs on one compute unit: 24.8 us, where
+// the merge on many units takes 4.2 and this kernel 3.9 (8 sequences; the whole step 43.6 ->
+// 26.7 us, 1 sequence of 1000 keys 31.0 -> 11.6).
 template <class T>
-__global__ __launch_bounds__(256) void k_attn_merge_fp8(AttnArgs a, uint8_t *packed,
-                                                        float *scales) {
+__global__ __launch_bounds__(256) void k_attn_encode_fp8(AttnArgs a, uint8_t *packed,
+                                                         float *scales) {
   constexpr int kWaves = 4, kHeads = 32;
-  __shared__ float weights[kHeads][32];
   __shared__ float maxima[kWaves];
   const int seq = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   int n, first;
   if (!attn_window(a, seq, n, first))
     return; // block-uniform; the split kernel raised the flag
-  const int active = min(a.splits, (n + kKeys - 1) / kKeys);
   bool fine = true;
-  for (int head = wave; head < a.hq; head += kWaves) {
-    const float v =
-        lane < active ? a.lse[((size_t)seq * a.splits + lane) * a.hq + head] : -INFINITY;
-    const float mx = xor_max32(v);
-    const float w = lane < active ? expf(v - mx) : 0.f;
-    const float total = xor_sum32(w);
-    if (lane < active) {
-      weights[head][lane] = w / total;
-      fine = fine && isfinite(weights[head][lane]);
-    }
-  }
-  __syncthreads();
   uint32_t words[kHeads / kWaves];
   float amax = 0.f;
 #pragma unroll
   for (int k = 0; k < kHeads / kWaves; ++k) {
-    const int head = wave + kWaves * k;
-    words[k] = 0u;
-    if (head >= a.hq)
-      continue;
-    float s0 = 0.f, s1 = 0.f;
-    for (int sp = 0; sp < active; ++sp) {
-      const float2 p = *reinterpret_cast<const float2 *>(
-          a.partial + (((size_t)seq * a.splits + sp) * a.hq + head) * kD + 2 * lane);
-      s0 = __builtin_fmaf(weights[head][sp], p.x, s0);
-      s1 = __builtin_fmaf(weights[head][sp], p.y, s1);
+    const int head = min(wave + kWaves * k, a.hq - 1); // heads past the row repeat the last
+    const size_t o = ((size_t)seq * a.hq + head) * kD + 2 * lane;
+    if constexpr (std::is_same<T, uint16_t>::value) {
+      words[k] = static_cast<const uint32_t *>(a.out)[o / 2];
+    } else {
+      const float2 v = *reinterpret_cast<const float2 *>(static_cast<const float *>(a.out) + o);
+      words[k] = pack2(v.x, v.y); // BF16-exact
     }
-    const uint32_t word = pack2(s0, s1);
-    words[k] = word;
+  }
+#pragma unroll
+  for (int k = 0; k < kHeads / kWaves; ++k) {
+    const uint32_t word = words[k];
     fine = fine && ((word & 0x7f80u) != 0x7f80u) && ((word & 0x7f800000u) != 0x7f800000u);
     amax = fmaxf(amax, fmaxf(fabsf(lo16(word)), fabsf(hi16(word))));
-    const size_t o = ((size_t)seq * a.hq + head) * kD + 2 * lane;
-    if constexpr (std::is_same<T, uint16_t>::value)
-      static_cast<uint32_t *>(a.out)[o / 2] = word;
-    else
-      *reinterpret_cast<float2 *>(static_cast<float *>(a.out) + o) =
-          make_float2(lo16(word), hi16(word));
   }
   amax = xor_reduce<32>(amax, [](float x, float y) { return fmaxf(x, y); });
   if (lane == 0)
     maxima[wave] = amax;
-  const bool row_fine = !__syncthreads_or(!fine);
+  const bool row_fine = !__syncthreads_or(!fine); // (k_attn_merge raised the flag)
   amax = fmaxf(fmaxf(maxima[0], maxima[1]), fmaxf(maxima[2], maxima[3]));
-  if (!row_fine && threadIdx.x == 0)
-    raise_bad(a.bad);
   const float scale = amax == 0.f ? 1.f : amax / 448.f;
   const float inverse = 1.f / scale;
   if (threadIdx.x == 0)
@@ -1145,26 +1155,34 @@ template <int G> __global__ __launch_bounds__(256) void k_q8_0_mx(AttnArgs a) {
 
 template <class T> __global__ __launch_bounds__(64) void k_q8_0_mx_merge(AttnArgs a) {
   const int head = blockIdx.x, seq = blockIdx.y, lane = threadIdx.x;
+  const size_t entry = (size_t)seq * a.splits * a.hq + head, step = (size_t)a.hq * kD;
+  const float *src = a.partial + entry * kD + 2 * lane;
+  const bool early = gridDim.x * gridDim.y <= kEarlyHeads;
+  const float lse = a.lse[entry + (size_t)min(lane & 31, a.splits - 1) * a.hq];
+  float2 p[kMaxSplits];
+  if (early)
+    merge_load(src, step, a.splits, p);
   int n, first;
   if (!attn_window(a, seq, n, first) || (a.local && a.cap != 1024))
     return; // the split kernel raised the flag
   // One entry per active split (at most 32: lanes 0..31).
   const int active = min(a.splits, (n + kQ8Tile - 1) / kQ8Tile), l32 = lane & 31;
-  const size_t base = (size_t)seq * a.splits;
-  const float v = l32 < active ? a.lse[(base + l32) * a.hq + head] : -INFINITY;
+  if (!early)
+    merge_load(src, step, active, p);
+  const float v = l32 < active ? lse : -INFINITY;
   float mxv = v;
   mxv = xor_max32(mxv);
-  const float p = isfinite(v) ? expf(v - mxv) : 0.f;
-  float den = p;
+  const float e = isfinite(v) ? expf(v - mxv) : 0.f;
+  float den = e;
   den = xor_sum32(den);
-  const float weight = p / den;
-  float x0 = 0.f, x1 = 0.f;
-  for (int sp = 0; sp < active; ++sp) {
-    const float w = __shfl(weight, sp, 64);
-    const float *src = a.partial + ((base + sp) * a.hq + head) * kD;
-    x0 = __builtin_fmaf(w, src[lane], x0);
-    x1 = __builtin_fmaf(w, src[64 + lane], x1);
-  }
+  const float weight = e / den;
+  float s0, s1;
+  merge_sum(p, weight, active, s0, s1);
+  // Lane l has features 2l, 2l + 1; the transforms take l and l + 64.
+  const int from = (lane >> 1), odd = lane & 1;
+  const float a0 = __shfl(s0, from, 64), a1 = __shfl(s1, from, 64);
+  const float b0 = __shfl(s0, from + 32, 64), b1 = __shfl(s1, from + 32, 64);
+  float x0 = odd ? a1 : a0, x1 = odd ? b1 : b0;
   // back from the V rotation: two 64-point transforms (features lane and lane + 64)
   hadamard64_pair(x0, x1, lane);
   x0 *= .125f;
@@ -1350,10 +1368,9 @@ int decode_attention(void *stream, const void *q, const padra_KVCache *kv, void 
       split_w(std::true_type{});
     else
       split_w(std::false_type{});
+    hipLaunchKernelGGL((k_attn_merge<T>), merge_grid, dim3(64), 0, s, a);
     if (fp8)
-      hipLaunchKernelGGL((k_attn_merge_fp8<T>), dim3(seqs), dim3(256), 0, s, a, packed, scales);
-    else
-      hipLaunchKernelGGL((k_attn_merge<T>), merge_grid, dim3(64), 0, s, a);
+      hipLaunchKernelGGL((k_attn_encode_fp8<T>), dim3(seqs), dim3(256), 0, s, a, packed, scales);
     return launched("DecodeAttention");
   };
   return act == PADRA_ACT_BF16 ? launch(uint16_t{}) : launch(float{});
