@@ -37,9 +37,9 @@ using namespace padra;
 namespace {
 
 constexpr int kD = 128, kKeys = 32;
-// Launches of up to this many sequences on a global cache order their split waves by
-// window length (the ranking reads seqs^2 control records).
-constexpr int kOrderMaxSeqs = 512, kRankMaxSeqs = 64;
+// Launches of up to this many sequences on a global cache order their splits by window
+// length (the ranking reads seqs^2 control records); up to kRankMaxSeqs in the split kernels.
+constexpr int kOrderMaxSeqs = 512, kRankMaxSeqs = 16;
 constexpr float kScoreScale = .08838834764831845f;
 
 int launched(const char *what) {
@@ -66,11 +66,12 @@ struct AttnArgs {
   int8_t *qcodes;
   float *qscale;
   const float *kvscales; // q8 caches: (k, v) scale pair per row and KV head
-  // The split kernels' sequence for grid slot z (longest window first), or null for
-  // slot z = sequence z.
+  // How a split kernel's workgroup finds its unit (sequence and split): kPlain, from the grid
+  // (every sequence's every split); otherwise unit blockIdx.y of the splits that have tiles,
+  // longest windows first: kRanked, each wave ranks the sequences itself; kOrdered, from `order`,
+  // written by an earlier kernel: the sequence of each rank, and its first unit << 9.
+  enum { kPlain, kRanked, kOrdered } units;
   int *order;
-  // Each split wave ranks the sequences itself (at most 64 of them, one per lane).
-  int rank;
 };
 
 // The sequence's admission and key window (Admitted, attention_gqa8_fragment_validation.cuh:
@@ -84,51 +85,129 @@ __device__ __forceinline__ bool attn_window(const AttnArgs &a, int seq, int &n, 
   return ok;
 }
 
-// Sequence `seq`'s place in the split kernels' dispatch order, written by a 64-lane block:
-// windows by decreasing length (a sequence that is not admitted counts as 0 keys), ties
-// by sequence index.  The split kernels give grid slot z to order[z], so the longest
-// windows start first and the shortest fill the end of the launch; every output is the
-// same as in sequence order.
-__device__ __forceinline__ void attn_rank(const AttnArgs &a, int seq) {
-  int n, first;
-  const int mine = attn_window(a, seq, n, first) ? n : 0;
-  int before = 0;
-  for (int j = threadIdx.x; j < a.seqs; j += 64) {
-    const int other = attn_window(a, j, n, first) ? n : 0;
-    before += other > mine || (other == mine && j < seq);
-  }
-  before = xor_reduce<32>(before, [](int x, int y) { return x + y; });
-  if (threadIdx.x == 0)
-    a.order[before] = seq;
+// A split kernel's unit of work: one split of one sequence's window.
+struct AttnUnit {
+  int seq, split, n, first; // the window: n keys from position `first`
+  int begin, end;           // the split's tiles
+};
+
+// The splits of an n-key window that have tiles (of TILE keys), and a unit's tiles.
+template <int TILE> __device__ __forceinline__ int attn_active(const AttnArgs &a, int n) {
+  return min(a.splits, (n + TILE - 1) / TILE);
 }
-// The split kernels' sequence for grid slot blockIdx.z, its admission and key window.  With
-// a.rank each wave ranks the sequences itself, one a lane: 0.1-0.5 us of its time against
-// a launch of its own for k_attn_order, whose 4.3 us (2 of them not hidden) every step paid.
-__device__ __forceinline__ bool attn_pick(const AttnArgs &a, int &seq, int &n, int &first) {
-  const int slot = blockIdx.z;
-  if (!a.rank) {
-    seq = a.order ? __builtin_amdgcn_readfirstlane(a.order[slot]) : slot;
-    return attn_window(a, seq, n, first);
+template <int TILE> __device__ __forceinline__ void attn_tiles(const AttnArgs &a, AttnUnit &x) {
+  const int tiles = (x.n + TILE - 1) / TILE, active = min(a.splits, tiles);
+  x.begin = tiles * x.split / active;
+  x.end = tiles * (x.split + 1) / active;
+}
+template <int TILE> __device__ __forceinline__ bool attn_admitted(const AttnArgs &a, int seq,
+                                                                  int &n, int &first) {
+  return attn_window(a, seq, n, first) && !(TILE == 128 && a.local && a.cap != 1024);
+}
+
+// The unit of (sequence, split), false where the split has no tile.  `raise`: whether this
+// thread reports a sequence that is not admitted.
+template <int TILE> __device__ __forceinline__ bool attn_unit(const AttnArgs &a, int seq, int split,
+                                                              bool raise, AttnUnit &x) {
+  x.seq = seq;
+  x.split = split;
+  if (!attn_admitted<TILE>(a, x.seq, x.n, x.first)) {
+    if (split == 0 && raise)
+      raise_bad(a.bad);
+    return false;
   }
+  if (split >= attn_active<TILE>(a, x.n))
+    return false;
+  attn_tiles<TILE>(a, x);
+  return true;
+}
+
+// Unit u among all the batch's splits that have tiles, the longest windows' first (ties by
+// sequence), so that the longest start first and the shortest fill the end of the launch.  The
+// units past the last active one are the end of the grid.  Where each sequence's
+// inactive splits (all but n / 32 of 32) came between the others' active ones, their waves, which
+// do no more than read the control records, held the slots: 64 sequences of up to 300 keys
+// (BF16) 40.4 -> 26.2 us, of up to 1000 keys (q8_0) 83.7 -> 33.9 us.
+//
+// In the split kernels (2 to 16 sequences, one a lane): saves the launch of k_attn_order, 2-4 us,
+// and costs each wave 5 instructions a sequence; at 64 sequences those were 7 us of
+// 111 (8000 keys).
+template <int TILE> __device__ __forceinline__ bool attn_unit_ranked(const AttnArgs &a, int u,
+                                                                     bool raise, AttnUnit &x) {
   const int lane = threadIdx.x & 63;
-  int mine = 0, from = 0;
-  bool ok = false;
-  if (lane < a.seqs)
-    ok = attn_window(a, lane, mine, from);
-  // window length (0 if not admitted), then the lower index: distinct keys
-  const int key = lane < a.seqs ? ((ok ? mine : 0) << 6) + 63 - lane : -1;
-  int before = 0;
+  int n = 0, first = 0;
+  const bool ok = lane < a.seqs && attn_admitted<TILE>(a, lane, n, first);
+  if (u == 0 && __ballot(lane < a.seqs && !ok) != 0 && raise)
+    raise_bad(a.bad);
+  const int active = ok ? attn_active<TILE>(a, n) : 0;
+  const int key = ((ok ? n : 0) << 6) + 63 - lane; // distinct
+  int before = 0;                                  // active splits of longer windows
   for (int j = 0; j < a.seqs; j += 8)
 #pragma unroll
     for (int i = 0; i < 8; ++i)
-      before += __builtin_amdgcn_readlane(key, j + i) > key;
-  seq = (int)__builtin_ctzll(__ballot(lane < a.seqs && before == slot));
-  n = __builtin_amdgcn_readlane(mine, seq);
-  first = __builtin_amdgcn_readlane(from, seq);
-  return __builtin_amdgcn_readlane((int)ok, seq) != 0;
+      before += __builtin_amdgcn_readlane(key, j + i) > key
+                    ? __builtin_amdgcn_readlane(active, j + i)
+                    : 0;
+  const uint64_t mine = __ballot(before <= u && u < before + active);
+  if (mine == 0)
+    return false; // wave-uniform
+  x.seq = (int)__builtin_ctzll(mine);
+  x.split = u - __builtin_amdgcn_readlane(before, x.seq);
+  x.n = __builtin_amdgcn_readlane(n, x.seq);
+  x.first = __builtin_amdgcn_readlane(first, x.seq);
+  attn_tiles<TILE>(a, x);
+  return true;
 }
 
-__global__ __launch_bounds__(64) void k_attn_order(AttnArgs a) { attn_rank(a, blockIdx.x); }
+// More sequences: ranked by an earlier kernel, a 64-lane block per sequence.
+template <int TILE> __device__ __forceinline__ void attn_rank(const AttnArgs &a, int seq) {
+  int n, first;
+  const bool ok = attn_admitted<TILE>(a, seq, n, first);
+  if (!ok && threadIdx.x == 0)
+    raise_bad(a.bad);
+  const int mine = ok ? n : 0;
+  int before = 0, units = 0;
+  for (int j = threadIdx.x; j < a.seqs; j += 64) {
+    const int other = attn_admitted<TILE>(a, j, n, first) ? n : 0;
+    if (other > mine || (other == mine && j < seq)) {
+      ++before;
+      units += attn_active<TILE>(a, other);
+    }
+  }
+  const auto sum = [](int x, int y) { return x + y; };
+  before = xor_reduce<32>(before, sum);
+  units = xor_reduce<32>(units, sum);
+  if (threadIdx.x == 0)
+    a.order[before] = seq | (units << 9);
+}
+template <int TILE> __device__ __forceinline__ bool attn_unit_ordered(const AttnArgs &a, int u,
+                                                                      AttnUnit &x) {
+  int entry = 0; // of the last rank whose first unit is u or before (rank 0's is 0)
+  for (int j = 0; j < a.seqs; j += 64) {
+    const int rank = j + (threadIdx.x & 63);
+    const int e = a.order[min(rank, a.seqs - 1)];
+    const uint64_t m = __ballot(rank < a.seqs && (e >> 9) <= u);
+    if (m != 0)
+      entry = __builtin_amdgcn_readlane(e, 63 - (int)__builtin_clzll(m));
+  }
+  return attn_unit<TILE>(a, entry & 511, u - (entry >> 9), false, x);
+}
+
+// A workgroup's unit; `raise` as above.
+template <int TILE> __device__ __forceinline__ bool attn_find(const AttnArgs &a, bool raise,
+                                                              AttnUnit &x) {
+  if (a.units == AttnArgs::kPlain)
+    return attn_unit<TILE>(a, blockIdx.z, blockIdx.y, raise, x);
+  if (a.units == AttnArgs::kRanked)
+    return attn_unit_ranked<TILE>(a, blockIdx.y, raise, x);
+  return attn_unit_ordered<TILE>(a, blockIdx.y, x);
+}
+
+constexpr int kQ8Tile = 128, kRowBytes = 544; // q8_0: keys of a tile, bytes of a row
+
+__global__ __launch_bounds__(64) void k_attn_order(AttnArgs a) {
+  attn_rank<kKeys>(a, blockIdx.x);
+}
 
 // Hadamard stages on lane bits 0..5, bit 0 first, of two values per lane.
 __device__ __forceinline__ void hadamard64_pair(float &x0, float &x1, int lane) {
@@ -265,19 +344,23 @@ __global__ __launch_bounds__(64 * W) void k_attn_mx(AttnArgs a) {
   __shared__ __align__(16) uint2 vq[W][kKeys / 4][kD];
   __shared__ __align__(16) uint4 pq[W][64];
   __shared__ __align__(16) float tile_max[W][16], tile_alpha[W][16], tile_total[W][16];
-  const int split = blockIdx.x, kv = blockIdx.y, lane = threadIdx.x & 63;
+  const int lane = threadIdx.x & 63;
   const int wave = W == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int col = lane & 15, grp = lane >> 4;
-  int seq, n, first;
-  if (!attn_pick(a, seq, n, first)) {
-    if (split == 0 && kv == 0 && threadIdx.x == 0)
-      raise_bad(a.bad);
-    return;
-  }
-  const int tiles = (n + kKeys - 1) / kKeys, active = min(a.splits, tiles);
-  if (split >= active)
+  AttnUnit unit;
+  if (!attn_find<kKeys>(a, blockIdx.x == 0 && threadIdx.x == 0, unit))
     return; // block-uniform
-  const int begin = tiles * split / active, end = tiles * (split + 1) / active;
+  int kv = blockIdx.x;
+  if (a.units == AttnArgs::kOrdered) {
+    // In a large batch a sequence's workgroups go head by head, each head's splits in a row:
+    // 64 sequences of 32768 keys (BF16) 360 us, with the heads of a split side by side 370.
+    const int active = attn_active<kKeys>(a, unit.n), at = unit.split * a.hkv + kv;
+    kv = at / active;
+    unit.split = at - kv * active;
+    attn_tiles<kKeys>(a, unit);
+  }
+  const int seq = unit.seq, split = unit.split, n = unit.n, first = unit.first;
+  const int begin = unit.begin, end = unit.end;
   const int features = a.hkv * kD;
   constexpr int ES = Q8 ? 1 : 2; // bytes per cache element
   const size_t head_off = ((size_t)seq * a.seq_stride * features + kv * kD) * ES;
@@ -726,12 +809,10 @@ __global__ __launch_bounds__(256) void k_attn_encode_fp8(AttnArgs a, uint8_t *pa
 // Here (k_q8_0_mx) each stream is its own partial entry and the merge joins the 4 * splits
 // entries; scores and PV run on the matrix cores.
 
-constexpr int kQ8Tile = 128, kRowBytes = 544;
-
 template <class T> __global__ __launch_bounds__(64) void k_q8_0_query(AttnArgs a) {
   const int head = blockIdx.x, seq = blockIdx.y, lane = threadIdx.x;
-  if (a.order && head == 0) // the split kernel's dispatch order, one sequence per block
-    attn_rank(a, seq);
+  if (a.units == AttnArgs::kOrdered && head == 0) // one sequence per block
+    attn_rank<kQ8Tile>(a, seq);
   const size_t base = ((size_t)seq * a.hq + head) * kD;
   float x0 = act_value<T>(a.q, base + lane), x1 = act_value<T>(a.q, base + 64 + lane);
   if (__ballot(!isfinite(x0) || !isfinite(x1)) != 0) {
@@ -828,23 +909,22 @@ template <int G> __global__ __launch_bounds__(256) void k_q8_0_mx(AttnArgs a) {
   __shared__ float ksc_all[4][32][4];    // K block scales by key
   __shared__ float vsc_all[4][4][32];    // V block scales by block
   __shared__ float ps_all[4][8][36];     // probabilities by head (rows padded)
-  const int split = blockIdx.x, tid = threadIdx.x, kv = tid >> 6;
+  const int tid = threadIdx.x, kv = tid >> 6;
   const int lane = tid & 63, col = lane & 15, grp = lane >> 4;
   auto &kq = kq_all[kv].r;
   auto &vq = vq_all[kv].r;
   auto &ksc = ksc_all[kv];
   auto &vsc = vsc_all[kv];
   auto &ps = ps_all[kv];
-  int seq, n, first;
-  if (!attn_pick(a, seq, n, first) || (a.local && a.cap != 1024)) {
-    if (split == 0 && tid == 0)
-      raise_bad(a.bad);
-    return;
-  }
-  const int tiles = (n + kQ8Tile - 1) / kQ8Tile, active = min(a.splits, tiles);
-  if (split >= active)
+  AttnUnit unit;
+  if (!attn_find<kQ8Tile>(a, tid == 0, unit))
     return; // block-uniform
-  const int begin = tiles * split / active, end = tiles * (split + 1) / active;
+  const int seq = __builtin_amdgcn_readfirstlane(unit.seq);
+  const int split = __builtin_amdgcn_readfirstlane(unit.split);
+  const int n = __builtin_amdgcn_readfirstlane(unit.n);
+  const int first = __builtin_amdgcn_readfirstlane(unit.first);
+  const int begin = __builtin_amdgcn_readfirstlane(unit.begin);
+  const int end = __builtin_amdgcn_readfirstlane(unit.end);
   const int features = a.hkv * kD, dbytes = 2 * (features / 32);
   const uint8_t *krows = static_cast<const uint8_t *>(static_cast<const void *>(a.kc)) +
                          (size_t)seq * a.seq_stride * kRowBytes;
@@ -1293,12 +1373,13 @@ int decode_attention(void *stream, const void *q, const padra_KVCache *kv, void 
   a.lse = scratch + entries * kD;
   a.qcodes = reinterpret_cast<int8_t *>(scratch + qbase);
   a.qscale = scratch + qbase + (long long)seqs * q_heads * (kD / 4);
-  // Longest windows first when the lengths can differ much: several sequences on a
-  // global cache (a local ring's windows are at most 1024 keys).
+  // Units longest first, without the inactive ones, when the lengths can differ much: several
+  // sequences on a global cache (a local ring's windows are at most 1024 keys).
   const long long obase = qbase + (q8 ? (long long)seqs * q_heads * (kD / 4 + 4) : 0);
-  const bool ordered = seqs >= 2 && seqs <= kOrderMaxSeqs && !local;
-  a.rank = ordered && seqs <= kRankMaxSeqs && !q8; // (q8_0's query kernel ranks them)
-  a.order = ordered && !a.rank ? reinterpret_cast<int *>(scratch + obase) : nullptr;
+  a.order = reinterpret_cast<int *>(scratch + obase);
+  a.units = seqs < 2 || seqs > kOrderMaxSeqs || local ? AttnArgs::kPlain
+            : seqs <= kRankMaxSeqs                    ? AttnArgs::kRanked
+                                                      : AttnArgs::kOrdered;
   a.decode = pos->decode;
   a.seqs = seqs;
   a.hq = q_heads;
@@ -1313,28 +1394,33 @@ int decode_attention(void *stream, const void *q, const padra_KVCache *kv, void 
   a.bad = bad;
   a.kvscales = static_cast<const float *>(kv->scales);
   const hipStream_t s = static_cast<hipStream_t>(stream);
-  const dim3 split_grid(splits, kv_heads, seqs), merge_grid(q_heads, seqs);
+  // The heads of a split side by side: with the heads outermost each would bring its own tail
+  // of inactive splits (8 sequences of 8000 keys 24.1 -> 25.9 us).
+  const bool plain = a.units == AttnArgs::kPlain;
+  const dim3 split_grid = plain ? dim3(kv_heads, splits, seqs) : dim3(kv_heads, splits * seqs);
+  const dim3 q8_grid = plain ? dim3(1, splits, seqs) : dim3(1, splits * seqs);
+  const dim3 merge_grid(q_heads, seqs);
   const int group = q_heads / kv_heads;
   if (group != 1 && group != 2 && group != 4 && group != 8)
     return PADRA_UNSUPPORTED;
   auto launch = [&](auto tag) -> int {
     using T = decltype(tag);
-    if (a.order && !q8) // (the q8_0 query kernel ranks the sequences itself)
+    if (a.units == AttnArgs::kOrdered && !q8) // (the q8_0 query kernel ranks them itself)
       hipLaunchKernelGGL(k_attn_order, dim3(seqs), dim3(64), 0, s, a);
     if (q8) {
       hipLaunchKernelGGL((k_q8_0_query<T>), merge_grid, dim3(64), 0, s, a);
       switch (group) {
       case 1:
-        hipLaunchKernelGGL((k_q8_0_mx<1>), dim3(splits, 1, seqs), dim3(256), 0, s, a);
+        hipLaunchKernelGGL((k_q8_0_mx<1>), q8_grid, dim3(256), 0, s, a);
         break;
       case 2:
-        hipLaunchKernelGGL((k_q8_0_mx<2>), dim3(splits, 1, seqs), dim3(256), 0, s, a);
+        hipLaunchKernelGGL((k_q8_0_mx<2>), q8_grid, dim3(256), 0, s, a);
         break;
       case 4:
-        hipLaunchKernelGGL((k_q8_0_mx<4>), dim3(splits, 1, seqs), dim3(256), 0, s, a);
+        hipLaunchKernelGGL((k_q8_0_mx<4>), q8_grid, dim3(256), 0, s, a);
         break;
       default:
-        hipLaunchKernelGGL((k_q8_0_mx<8>), dim3(splits, 1, seqs), dim3(256), 0, s, a);
+        hipLaunchKernelGGL((k_q8_0_mx<8>), q8_grid, dim3(256), 0, s, a);
         break;
       }
       hipLaunchKernelGGL((k_q8_0_mx_merge<T>), merge_grid, dim3(64), 0, s, a);

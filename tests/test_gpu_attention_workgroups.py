@@ -103,3 +103,58 @@ def test_decode_attention_rows_past_4gib():
         torch.cuda.synchronize()
         assert torch.equal(some, out[:, h:h + 4])
     assert bad.item() == 0
+
+
+@pytest.mark.parametrize("fmt", [abi.KV_BF16, abi.KV_Q8, abi.KV_Q8_0])
+@pytest.mark.parametrize("seqs", [2, 16, 17, 65])
+def test_decode_attention_units(fmt, seqs):
+    """Batches on either side of each way the split kernels find their work (2 to 16 sequences
+    ranked by the waves, 17 to 64 and 65 to 512 by a kernel before), with windows from one key to
+    the capacity, ties, and two sequences that are not admitted: those raise the flag and their
+    rows stay, every other row equals the sequence decoded alone."""
+    hq, hkv, cap = 8, 4, 2048
+    print(f"[case] attention units fmt={fmt} seqs={seqs}", flush=True)
+    rng = np.random.default_rng(7 * seqs + fmt)
+    positions = rng.integers(0, cap, seqs)
+    positions[:2] = cap - 1, 0
+    positions[2::3] = 100
+    q = torch.from_numpy(synth.bf16_bits(rng.standard_normal((seqs, hq, 128)).astype(np.float32))
+                         .view(np.int16)).cuda()
+    g = torch.Generator(device="cuda").manual_seed(seqs)
+    if fmt == abi.KV_BF16:
+        kc, vc = (torch.randn((seqs * cap, 512), generator=g, device="cuda").bfloat16()
+                  for _ in range(2))
+    else:
+        width = 544 if fmt == abi.KV_Q8_0 else 512
+        kc, vc = (torch.randint(-127, 128, (seqs * cap, width), generator=g, device="cuda",
+                                dtype=torch.int8) for _ in range(2))
+        if fmt == abi.KV_Q8_0:
+            for t in (kc, vc):
+                t[:, :32].view(torch.int16)[:] = 0x2400
+    sc = torch.rand((seqs * cap, hkv, 2), generator=g, device="cuda") * .01 + .01
+    states = torch.tensor([[5, p, cap, 10, p, min(p, 1024), 0, 0] for p in positions.tolist()],
+                          dtype=torch.int32)
+
+    def run(rows, st, out):
+        some = slice(rows.start * cap, rows.stop * cap)
+        bad = torch.zeros(1, dtype=torch.int32, device="cuda")
+        kv = ops.kv_cache(fmt, kc[some], vc[some], cap, seq_stride=cap,
+                          scales=sc[some] if fmt == abi.KV_Q8 else None)
+        ops.DecodeAttention(q[rows], kv, out, ops.positions_decode(st.cuda(), maximum=cap), bad,
+                            kv_heads=hkv)
+        torch.cuda.synchronize()
+        return bad.item()
+
+    alone = torch.empty((seqs, hq, 128), dtype=torch.int16, device="cuda")
+    for i in range(seqs):
+        assert run(slice(i, i + 1), states[i:i + 1], alone[i:i + 1]) == 0
+    out = torch.full_like(alone, 77)
+    assert run(slice(0, seqs), states, out) == 0
+    assert torch.equal(out, alone)
+    refused = {seqs - 1} if seqs == 2 else {0, seqs - 1}
+    for i in refused:
+        states[i, 7] = 1  # stopped
+    out.fill_(77)
+    assert run(slice(0, seqs), states, out) == 1
+    for i in range(seqs):
+        assert torch.equal(out[i], torch.full_like(out[i], 77) if i in refused else alone[i]), i
