@@ -809,36 +809,39 @@ __global__ __launch_bounds__(256) void k_attn_encode_fp8(AttnArgs a, uint8_t *pa
 // Here (k_q8_0_mx) each stream is its own partial entry and the merge joins the 4 * splits
 // entries; scores and PV run on the matrix cores.
 
-template <class T> __global__ __launch_bounds__(64) void k_q8_0_query(AttnArgs a) {
-  const int head = blockIdx.x, seq = blockIdx.y, lane = threadIdx.x;
-  if (a.units == AttnArgs::kOrdered && head == 0) // one sequence per block
-    attn_rank<kQ8Tile>(a, seq);
-  const size_t base = ((size_t)seq * a.hq + head) * kD;
-  float x0 = act_value<T>(a.q, base + lane), x1 = act_value<T>(a.q, base + 64 + lane);
-  if (__ballot(!isfinite(x0) || !isfinite(x1)) != 0) {
-    if (lane == 0)
-      raise_bad(a.bad);
-    return;
-  }
-  // features lane and lane + 64: stages on bits 0..5 across lanes, bit 6 in the lane
+// One query head's codes and block scales, by a wave: rotated features lane and lane + 64, of
+// blocks lane / 32 and 2 + lane / 32.  False (and nothing written) where a value is not finite.
+__device__ __forceinline__ bool q8_0_code_query(float x0, float x1, int lane, int8_t *codes,
+                                                float *scales) {
+  if (__ballot(!isfinite(x0) || !isfinite(x1)) != 0)
+    return false;
+  // stages on bits 0..5 across lanes, bit 6 in the lane
   hadamard64_pair(x0, x1, lane);
   const float y0 = (x0 + x1) * .08838834764831845f, y1 = (x0 - x1) * .08838834764831845f;
-  // blocks lane / 32 (feature lane) and 2 + lane / 32 (feature lane + 64)
   float m0 = fabsf(y0), m1 = fabsf(y1);
   m0 = xor_max32(m0);
   m1 = xor_max32(m1);
   const float d0 = m0 / 127.f, d1 = m1 / 127.f;
-  if (__ballot(!isfinite(d0) || !isfinite(d1)) != 0) {
-    if (lane == 0)
-      raise_bad(a.bad);
-    return;
-  }
-  a.qcodes[base + lane] = (int8_t)q8_0_code(y0, d0 == 0.f ? 0.f : 1.f / d0);
-  a.qcodes[base + 64 + lane] = (int8_t)q8_0_code(y1, d1 == 0.f ? 0.f : 1.f / d1);
+  if (__ballot(!isfinite(d0) || !isfinite(d1)) != 0)
+    return false;
+  codes[lane] = (int8_t)q8_0_code(y0, d0 == 0.f ? 0.f : 1.f / d0);
+  codes[64 + lane] = (int8_t)q8_0_code(y1, d1 == 0.f ? 0.f : 1.f / d1);
   if ((lane & 31) == 0) {
-    a.qscale[((size_t)seq * a.hq + head) * 4 + lane / 32] = d0;
-    a.qscale[((size_t)seq * a.hq + head) * 4 + 2 + lane / 32] = d1;
+    scales[lane / 32] = d0;
+    scales[2 + lane / 32] = d1;
   }
+  return true;
+}
+
+template <class T> __global__ __launch_bounds__(64) void k_q8_0_query(AttnArgs a) {
+  const int head = blockIdx.x, seq = blockIdx.y, lane = threadIdx.x;
+  if (a.units == AttnArgs::kOrdered && head == 0) // one sequence per block
+    attn_rank<kQ8Tile>(a, seq);
+  const size_t row = (size_t)seq * a.hq + head, base = row * kD;
+  if (!q8_0_code_query(act_value<T>(a.q, base + lane), act_value<T>(a.q, base + 64 + lane), lane,
+                          a.qcodes + base, a.qscale + row * 4) &&
+      lane == 0)
+    raise_bad(a.bad);
 }
 
 __device__ __forceinline__ float f16_bits(uint32_t h) {
@@ -1233,6 +1236,315 @@ template <int G> __global__ __launch_bounds__(256) void k_q8_0_mx(AttnArgs a) {
     raise_bad(a.bad);
 }
 
+// ---- q8_0 split for few sequences -------------------------------------------------------
+// k_q8_0_mx walks the four streams of a split one after the other, with a workgroup per (sequence,
+// split) and a wave per KV head: one sequence ran 32 workgroups, 128 waves in all.  Here a workgroup takes one (sequence, split, KV head) and its four waves
+// one stream each, so that four times the waves walk a quarter of the slices, without a
+// barrier on the way; then each wave folds one row of every head's streams.  The query is
+// coded here too, while the first slice is on its way, which saves that launch.  Every sum has the
+// order it has in k_q8_0_mx: the bits are the same.
+// A head's codes are a quarter of each 544-byte row, and the lines at its ends belong to two
+// heads: the four heads of a split go to one XCD (workgroup ids 8 apart), whose L2 then holds
+// them; the loads are ordinary ones for that.  With many workgroups the whole-row loads of
+// k_q8_0_mx are better (the line ends then come from HBM twice).  Steps, k_q8_0_query and
+// k_q8_0_mx -> this kernel (us, merge included; workgroups = splits x 4 x sequences):
+//   1 sequence, 1000 / 32768 / 131072 keys (128)  20.6 -> 10.3, 71.5 -> 22.9, 237.6 -> 60.2
+//   4 sequences, to 8000 keys (512)               29.8 -> 16.7
+//   8 sequences (1024); 64 local rings (1024)     31.4 -> 26.8, 30.9 -> 28.4
+//   16 sequences, 16 heads (2048)                 39.6 -> 41.4
+//   64 sequences, 32768 keys (8192)               245.9 -> 301.9
+constexpr int kStreamsMaxGroups = 1024;
+
+// An ordinary 16-byte load as one vector value (a struct copy put the array in scratch memory).
+__device__ __forceinline__ uint4 ld_cached(const uint8_t *p) {
+  const u32x4_t v = *reinterpret_cast<const u32x4_t *>(p);
+  return make_uint4(v.x, v.y, v.z, v.w);
+}
+
+template <class T> __global__ __launch_bounds__(256) void k_q8_0_streams(AttnArgs a) {
+  // Per wave: the slice's K codes (32 keys of 8 chunks, exchanged by key), then its V codes as
+  // BF16 (4 keys per dimension and group, at slot vq_slot<true>(d) ^ 16 flip(group)), then
+  // the stream's outputs; block scales; probabilities by head.
+  __shared__ __align__(16) uint2 image[kStreams][8][kD];
+  __shared__ __align__(16) float ksc_all[kStreams][32][4], vsc_all[kStreams][4][32];
+  __shared__ __align__(16) float ps_all[kStreams][8][36];
+  __shared__ float dsum_all[kStreams][8], lse_all[kStreams][8];
+  __shared__ __align__(16) int8_t qcodes[8][kD];
+  __shared__ float qscale[8][4];
+  const int lane = threadIdx.x & 63, s = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int col = lane & 15, grp = lane >> 4, G = a.group;
+  const int kv = blockIdx.x >> 3, u = 8 * blockIdx.y + (blockIdx.x & 7);
+  AttnUnit unit;
+  const bool raise = kv == 0 && threadIdx.x == 0;
+  if (a.units == AttnArgs::kRanked ? !attn_unit_ranked<kQ8Tile>(a, u, raise, unit)
+                                   : u >= a.seqs * a.splits ||
+                                         !attn_unit<kQ8Tile>(a, u / a.splits, u % a.splits, raise, unit))
+    return; // block-uniform
+  const int n = unit.n, head0 = kv * G;
+  const size_t head_off = 32 + kD * (size_t)kv, scale_off = 8 * (size_t)kv;
+  const uint8_t *krows = reinterpret_cast<const uint8_t *>(a.kc) +
+                         (size_t)unit.seq * a.seq_stride * kRowBytes;
+  const uint8_t *vrows = reinterpret_cast<const uint8_t *>(a.vc) +
+                         (size_t)unit.seq * a.seq_stride * kRowBytes;
+  uint4 *kq = reinterpret_cast<uint4 *>(&image[s][0][0]);
+  auto &vq = image[s];
+  auto &ksc = ksc_all[s];
+  auto &vsc = vsc_all[s];
+  auto &ps = ps_all[s];
+
+  // Slice loads: K load m is key lane / 8 + 8 m, codes 16 (lane % 8) ..; V load m is key
+  // 4 (lane / 8) + m; the four block scales of K row lane (lanes 0..31) or V row lane - 32.
+  // Window offsets past the last key read the last key's row; their scales are zeroed (the
+  // reference zero-fills both) and their scores masked.
+  const uint32_t first_row = (uint32_t)(unit.first % a.cap);
+  auto row_at = [&](int o) { // the window holds at most cap keys: one wrap
+    const uint32_t r = first_row + (uint32_t)min(o, n - 1);
+    return (size_t)min(r, r - (uint32_t)a.cap) * kRowBytes;
+  };
+  uint4 kw[4], vw[4];
+  uint2 hw;
+  auto load_slice = [&](int o0) {
+#pragma unroll
+    for (int m = 0; m < 4; ++m)
+      kw[m] = ld_cached(krows + row_at(o0 + (lane >> 3) + 8 * m) + head_off + 16 * (lane & 7));
+#pragma unroll
+    for (int m = 0; m < 4; ++m)
+      vw[m] = ld_cached(vrows + row_at(o0 + 4 * (lane >> 3) + m) + head_off + 16 * (lane & 7));
+    hw = *reinterpret_cast<const uint2 *>((lane < 32 ? krows : vrows) + row_at(o0 + (lane & 31)) +
+                                          scale_off);
+  };
+  // This wave's slices: keys 32 s .. 32 s + 31 of the split's tiles that lie in the window
+  // (a slice past it would leave every value as it is).
+  const int o_begin = unit.begin * kQ8Tile + 32 * s;
+  const int o_end = min(unit.end * kQ8Tile, n);
+  if (o_begin < o_end)
+    load_slice(o_begin);
+
+  bool fine = true;
+#pragma unroll
+  for (int k = 0; k < 2; ++k) { // wave s codes heads s and s + 4
+    const int h = s + 4 * k;
+    if (h < G) {
+      const size_t o = ((size_t)unit.seq * a.hq + head0 + h) * kD + lane;
+      fine = q8_0_code_query(act_value<T>(a.q, o), act_value<T>(a.q, o + 64), lane, qcodes[h],
+                             qscale[h]) &&
+             fine;
+    }
+  }
+  __syncthreads();
+  // Query A operands: row col = (head 4 j + col / 4, block col % 4); K-slot group grp of
+  // step h covers dimensions 64 h + 16 grp .. + 15, of block 2 h + grp / 2.
+  uint4 aq[2][2];
+  float qd[2][4]; // block scales of head 4 j + grp
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const int hh = 4 * j + (col >> 2);
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      aq[j][h] = make_uint4(0, 0, 0, 0);
+      if (hh < G && (col & 3) == 2 * h + (grp >> 1))
+        aq[j][h] = *reinterpret_cast<const uint4 *>(&qcodes[hh][64 * h + 16 * grp]);
+    }
+#pragma unroll
+    for (int b = 0; b < 4; ++b)
+      qd[j][b] = 4 * j + grp < G ? qscale[4 * j + grp][b] : 0.f;
+  }
+
+  float mx[2] = {-INFINITY, -INFINITY}, den[2][2] = {{0.f, 0.f}, {0.f, 0.f}};
+  f32x4_t o[8];
+#pragma unroll
+  for (int t = 0; t < 8; ++t)
+    o[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  // One slice; MORE: this wave's next one is loaded once the registers are free.
+  auto slice = [&](int o0, auto more) {
+    const uint4 va[4] = {vw[0], vw[1], vw[2], vw[3]};
+#pragma unroll
+    for (int m = 0; m < 4; ++m) {
+      const int key = (lane >> 3) + 8 * m;
+      kq[8 * key + ((lane & 7) ^ ((key >> 1) & 7))] = kw[m];
+    }
+    {
+      const bool inside = o0 + (lane & 31) < n;
+      const float4 d = make_float4(inside ? f16_bits(hw.x & 0xffffu) : 0.f,
+                                   inside ? f16_bits(hw.x >> 16) : 0.f,
+                                   inside ? f16_bits(hw.y & 0xffffu) : 0.f,
+                                   inside ? f16_bits(hw.y >> 16) : 0.f);
+      if (lane < 32) {
+        *reinterpret_cast<float4 *>(&ksc[lane][0]) = d;
+      } else {
+        vsc[0][lane - 32] = d.x;
+        vsc[1][lane - 32] = d.y;
+        vsc[2][lane - 32] = d.z;
+        vsc[3][lane - 32] = d.w;
+      }
+    }
+    if constexpr (decltype(more)::value) {
+      load_slice(o0 + kQ8Tile);
+      issue_point();
+    }
+    // Scores: head 4 j + grp, key 16 k + col.
+    float sc[2][2];
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      const uint4 b0 = kq[8 * (16 * k + col) + (grp ^ (col >> 1))];
+      const uint4 b1 = kq[8 * (16 * k + col) + ((4 + grp) ^ (col >> 1))];
+      const float4 kd = *reinterpret_cast<const float4 *>(&ksc[16 * k + col][0]);
+      const bool valid = o0 + 16 * k + col < n;
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        i32x4_t d = mfma_i8(aq[j][0], b0, i32x4_t{0, 0, 0, 0});
+        d = mfma_i8(aq[j][1], b1, d);
+        float dot = 0.f;
+        dot = __builtin_fmaf((float)d[0], kd.x * qd[j][0], dot);
+        dot = __builtin_fmaf((float)d[1], kd.y * qd[j][1], dot);
+        dot = __builtin_fmaf((float)d[2], kd.z * qd[j][2], dot);
+        dot = __builtin_fmaf((float)d[3], kd.w * qd[j][3], dot);
+        sc[k][j] = valid ? dot * kScoreScale : -INFINITY;
+      }
+    }
+    // V takes the K codes' place (a wave's LDS accesses run in program order).
+    {
+      float f[4][16];
+#pragma unroll
+      for (int m = 0; m < 4; ++m) {
+        const uint32_t w[4] = {va[m].x, va[m].y, va[m].z, va[m].w};
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int b = 0; b < 4; ++b)
+            f[m][4 * i + b] = (float)(int8_t)((w[i] >> (8 * b)) & 0xffu);
+      }
+      const int t7 = lane & 7, j = lane >> 3;
+      uint2 *dst = &vq[j][(16 * t7) ^ (((j ^ (j >> 1)) & 1) << 4)];
+#pragma unroll
+      for (int e = 0; e < 16; e += 2)
+        *reinterpret_cast<uint4 *>(dst + 2 * ((e / 2 + t7) & 7)) =
+            make_uint4(pack2(f[0][e], f[1][e]), pack2(f[2][e], f[3][e]),
+                       pack2(f[0][e + 1], f[1][e + 1]), pack2(f[2][e + 1], f[3][e + 1]));
+    }
+    float alpha[2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const float next = fmaxf(mx[j], row_max16(fmaxf(sc[0][j], sc[1][j])));
+      alpha[j] = isfinite(mx[j]) ? __expf(mx[j] - next) : 0.f;
+      mx[j] = next;
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        const float p = isfinite(sc[k][j]) ? __expf(sc[k][j] - next) : 0.f;
+        den[k][j] = __builtin_fmaf(den[k][j], alpha[j], p);
+        ps[4 * j + grp][16 * k + col] = p;
+      }
+    }
+    // Rows 4 grp + i of the PV accumulators are head (4 grp + i) % 8, whose alpha lane 16 i
+    // holds (alpha[0] for heads 0..3, alpha[1] for 4..7).
+    if (__ballot(alpha[0] != 1.f || alpha[1] != 1.f) != 0) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float a0 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(alpha[0]), 16 * i));
+        const float a1 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(alpha[1]), 16 * i));
+        const float ar = (grp & 1) ? a1 : a0;
+#pragma unroll
+        for (int t = 0; t < 8; ++t)
+          o[t][i] *= ar;
+      }
+    }
+    // PV A operands: row col = (head col % 8, block 2 c + col / 8); K-slots of group grp are
+    // keys 8 grp .. 8 grp + 7.
+    uint4 ahi[2], alo[2];
+    {
+      const int hh = col & 7;
+      const float4 p0 = *reinterpret_cast<const float4 *>(&ps[hh][8 * grp]);
+      const float4 p1 = *reinterpret_cast<const float4 *>(&ps[hh][8 * grp + 4]);
+      const float pv[8] = {p0.x, p0.y, p0.z, p0.w, p1.x, p1.y, p1.z, p1.w};
+#pragma unroll
+      for (int c = 0; c < 2; ++c) {
+        const int b = 2 * c + (col >> 3);
+        const float4 v0 = *reinterpret_cast<const float4 *>(&vsc[b][8 * grp]);
+        const float4 v1 = *reinterpret_cast<const float4 *>(&vsc[b][8 * grp + 4]);
+        const float vv[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
+        uint32_t hi[4], lo[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float f0 = hh < G ? pv[2 * e] * vv[2 * e] : 0.f;
+          const float f1 = hh < G ? pv[2 * e + 1] * vv[2 * e + 1] : 0.f;
+          bf16_split2(f0, f1, hi[e], lo[e]);
+        }
+        ahi[c] = make_uint4(hi[0], hi[1], hi[2], hi[3]);
+        alo[c] = make_uint4(lo[0], lo[1], lo[2], lo[3]);
+      }
+    }
+#pragma unroll
+    for (int t = 0; t < 8; ++t) {
+      const int d = vq_slot<true>(16 * t + col) ^ ((grp & 1) << 4);
+      const uint2 v0 = vq[2 * grp][d], v1 = vq[2 * grp + 1][d ^ 16];
+      const uint4 bv = make_uint4(v0.x, v0.y, v1.x, v1.y);
+      o[t] = mfma_bf16(ahi[t >> 2], bv, o[t]);
+      o[t] = mfma_bf16(alo[t >> 2], bv, o[t]);
+    }
+  };
+  int o0 = o_begin;
+  for (; o0 + kQ8Tile < o_end; o0 += kQ8Tile)
+    slice(o0, std::true_type{});
+  if (o0 < o_end)
+    slice(o0, std::false_type{});
+
+  // Each stream's log-sum-exp (den over the 32 key positions) and outputs, for the fold.
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const float dsum = row_sum16(den[0][j] + den[1][j]);
+    if (col == 0) {
+      dsum_all[s][4 * j + grp] = dsum;
+      lse_all[s][4 * j + grp] = dsum > 0.f ? mx[j] + logf(dsum) : -INFINITY;
+    }
+  }
+  float *out = reinterpret_cast<float *>(&image[s][0][0]); // [8 tiles][4 rows][64 lanes]
+#pragma unroll
+  for (int t = 0; t < 8; ++t)
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      out[64 * (4 * t + i) + lane] = o[t][i];
+  __syncthreads();
+  // Wave i = s folds row i of the PV layout (head (4 grp + i) % 8) over the streams in order,
+  // with weight exp(lse - max), for this lane's four dimension tiles t = 4 u + 2 (grp / 2) + v;
+  // streams without a finite log-sum-exp carry no weight.
+  const int i = s, hh = (4 * grp + i) & 7;
+  float cm = -INFINITY, ct = 0.f, cs[4] = {0.f, 0.f, 0.f, 0.f};
+  bool has = false;
+  for (int st = 0; st < kStreams; ++st) {
+    const float d = dsum_all[st][hh], l = lse_all[st][hh];
+    const float *from = reinterpret_cast<const float *>(&image[st][0][0]) + 64 * i + lane;
+    float x[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      x[k] = from[256 * (4 * (k >> 1) + 2 * (grp >> 1) + (k & 1))];
+    if (isfinite(l)) {
+      has = true;
+      const float m2 = fmaxf(cm, l);
+      const float wa = isfinite(cm) ? expf(cm - m2) : 0.f, wb = expf(l - m2);
+      ct = __builtin_fmaf(ct, wa, wb);
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+        cs[k] = __builtin_fmaf(cs[k], wa, wb * (x[k] / d));
+      cm = m2;
+    }
+  }
+  // The split's entry: the combined output and log-sum-exp of each head.
+  const size_t entry = (size_t)unit.seq * a.splits + unit.split;
+  if (hh < G) {
+    float *dst = a.partial + (entry * a.hq + head0 + hh) * kD + col;
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      dst[16 * (4 * (k >> 1) + 2 * (grp >> 1) + (k & 1))] = ct > 0.f ? cs[k] / ct : 0.f;
+    if (col == 0 && grp < 2)
+      a.lse[entry * a.hq + head0 + hh] = ct > 0.f ? cm + logf(ct) : -INFINITY;
+    // The reference's check of the split's combined weight: it fails when no stream of a
+    // head has a finite log-sum-exp (a stream's is finite or -inf).
+    fine = fine && has;
+  }
+  if (__ballot(!fine) != 0 && lane == 0)
+    raise_bad(a.bad);
+}
+
 template <class T> __global__ __launch_bounds__(64) void k_q8_0_mx_merge(AttnArgs a) {
   const int head = blockIdx.x, seq = blockIdx.y, lane = threadIdx.x;
   const size_t entry = (size_t)seq * a.splits * a.hq + head, step = (size_t)a.hq * kD;
@@ -1407,6 +1719,12 @@ int decode_attention(void *stream, const void *q, const padra_KVCache *kv, void 
     using T = decltype(tag);
     if (a.units == AttnArgs::kOrdered && !q8) // (the q8_0 query kernel ranks them itself)
       hipLaunchKernelGGL(k_attn_order, dim3(seqs), dim3(64), 0, s, a);
+    if (q8 && splits * kv_heads * seqs <= kStreamsMaxGroups) {
+      hipLaunchKernelGGL((k_q8_0_streams<T>), dim3(8 * kv_heads, (splits * seqs + 7) / 8), dim3(256),
+                         0, s, a);
+      hipLaunchKernelGGL((k_q8_0_mx_merge<T>), merge_grid, dim3(64), 0, s, a);
+      return launched("DecodeAttention");
+    }
     if (q8) {
       hipLaunchKernelGGL((k_q8_0_query<T>), merge_grid, dim3(64), 0, s, a);
       switch (group) {

@@ -6,7 +6,7 @@ import torch
 
 from padra_amd import abi, ops, synth
 
-from attn_tolerance import attn_close, bound_bf16
+from attn_tolerance import attn_close, bound_bf16, bound_q8_0
 
 pytestmark = pytest.mark.gpu
 
@@ -24,15 +24,20 @@ def _rows(fmt, rng, rows):
     """A cache plane as stored: BF16 bits, or codes."""
     if fmt == abi.KV_BF16:
         return synth.bf16_bits(rng.standard_normal((rows, 512)).astype(np.float32)).view(np.int16)
-    return rng.integers(-127, 128, (rows, 512)).astype(np.int8)
+    if fmt == abi.KV_Q8:
+        return rng.integers(-127, 128, (rows, 512)).astype(np.int8)
+    out = rng.integers(-127, 128, (rows, 544)).astype(np.int8).view(np.uint8)
+    out[:, :32] = rng.uniform(.005, .02, (rows, 16)).astype(np.float16).view(np.uint8)
+    return out
 
 
-@pytest.mark.parametrize("fmt", [abi.KV_BF16, abi.KV_Q8])
+@pytest.mark.parametrize("fmt", [abi.KV_BF16, abi.KV_Q8, abi.KV_Q8_0])
 @pytest.mark.parametrize("local", [False, True])
 def test_decode_attention_workgroup_sizes(oracle, fmt, local):
     """17 sequences of 1 to 4096 keys (tile and round edges; local rings that wrap inside a
     tile), run in batches of 17 (one wave a split), 8 (two), 3 (four) and 1 (eight); 32 query
-    heads on 4 KV heads, 32 splits (local: 16, so batches of 17, 12, 6 and 1: one, one, four, eight)."""
+    heads on 4 KV heads, 32 splits (local: 16, so batches of 17, 12, 6 and 1: one, one, four, eight).
+    q8_0: a workgroup per split (batches of 17), or per split and KV head."""
     hq, hkv, capacity = 32, 4, 4096
     cap = 1024 if local else capacity
     windows = [1, 31, 32, 33, 64, 255, 256, 257, 1023, 1024, 1025, 1500, 2047, 2049, 4000, 4095,
@@ -68,6 +73,12 @@ def test_decode_attention_workgroup_sizes(oracle, fmt, local):
         assert np.array_equal(got, outs[0])
     for s in (0, 3, 7, 10, 16):
         k, v = kc[s * cap:(s + 1) * cap], vc[s * cap:(s + 1) * cap]
+        if fmt == abi.KV_Q8_0:
+            want, used, wbad = oracle.decode_attention_q8_0(q[s], k, v, windows[s] - 1, local=local)
+            bound = bound_q8_0(q[s], k, v, windows[s] - 1, local, used)
+            close, d = attn_close(outs[0][s], want, bound)
+            assert not wbad and close.all(), (windows[s], int(d.max()))
+            continue
         if fmt == abi.KV_BF16:
             k, v = k.view(np.uint16), v.view(np.uint16)
         else:
