@@ -615,9 +615,8 @@ int chain(hipStream_t s, const uint16_t *gather, int vocab, const int32_t *ids, 
 } // namespace
 
 namespace {
-// The chain on fp32 activations (the reference's buffers): up to head_wave_tokens one
-// launch of norm-row waves and per-head Q/K waves; above, the residual-norm launch, then
-// the four-lanes-per-head Q/K launch.
+// The chain on fp32 activations (the reference's buffers), in one launch: up to
+// head_wave_tokens of norm-row waves and per-head Q/K waves.
 int chain_f32(hipStream_t s, void *x, const void *residual, void *normalized,
               const uint16_t *gamma, int hidden, int tree, float *statistics, void *q, void *k,
               const void *v, const uint16_t *qn, const uint16_t *kn, const uint16_t *table,
@@ -652,18 +651,18 @@ int chain_f32(hipStream_t s, void *x, const void *residual, void *normalized,
                            dim3((unsigned)waves), dim3(64), 0, s, n, a, norm_waves, waves);
         return launched();
       }
-      // Larger launches run the two halves as two kernels on the stream: one kernel would
-      // give its norm rows the Q/K waves' registers (142 VGPRs, 3 waves per SIMD, against
-      // 89 and 5 for the norm rows alone); config 1: 22.1 us in one kernel, 11.4 + 9.8 us
-      // as two.
-      hipLaunchKernelGGL((k_norm<vt.value, j.value, float, true>), dim3((unsigned)norm_waves),
-                         dim3(64), 0, s, n);
-      const int st2 = launched();
-      if (st2)
-        return st2;
-      hipLaunchKernelGGL((k_qk<float, fmt.value>),
-                         dim3((unsigned)qk_wave_count<fmt.value>(tokens, q_heads, kv_heads)),
-                         dim3(64), 0, s, a);
+      // Above, one launch too, norm rows and then four-lanes-per-head Q/K waves.  The norm rows
+      // get the Q/K waves' registers there (142 VGPRs, 3 waves per SIMD, against 89 and 5
+      // alone), but the Q/K waves, whose chain alone lasts 6-7 us, start while the norm rows still
+      // stream.  One kernel against two on the stream (us; BF16 / q8 / rotated q8_0 cache):
+      //   hidden 2048, 16 heads, 512 tokens  8.7 : 11.9  11.8 : 14.7  11.3 : 14.5
+      //                         1000        13.7 : 14.9  15.6 : 17.2  15.2 : 16.9
+      //                         2048        22.8 : 22.7  24.1 : 25.4  25.0 : 26.5
+      //   hidden 2304, 32 heads, 512 tokens 10.1 : 13.2  12.5 : 15.5  12.1 : 15.3
+      //                         2048        30.2 : 33.4  31.4 : 34.7  31.7 : 35.0
+      const long long waves = norm_waves + qk_wave_count<fmt.value>(tokens, q_heads, kv_heads);
+      hipLaunchKernelGGL((k_chain<vt.value, j.value, fmt.value, false, float>),
+                         dim3((unsigned)waves), dim3(64), 0, s, n, a, norm_waves, waves);
       return launched();
     });
   });
