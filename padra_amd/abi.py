@@ -135,6 +135,26 @@ def lib() -> ctypes.CDLL:
     return _lib
 
 
+_fast = None
+
+
+def fast() -> dict:
+    """The entry points as functions of tensors (csrc/fastcall.cpp), bound to the library of
+    lib(): {name: function}."""
+    global _fast
+    if _fast is None:
+        lib()
+        path = os.path.join(_HERE, "_fastcall.so")
+        if not os.path.exists(path):
+            raise RuntimeError(f"{path} is missing: build it with `python -m padra_amd.build` "
+                               "(g++).  There is no fallback.")
+        import torch  # noqa: F401  (the libraries that _fastcall.so links)
+
+        from . import _fastcall
+        _fast = _fastcall.bind(library_path, PadraError)
+    return _fast
+
+
 def call(name: str, *args) -> None:
     status = getattr(lib(), name)(*args)
     if status != OK:

@@ -46,6 +46,34 @@ def command(out: str = OUT, asan: bool = False) -> list[str]:
            [os.path.join(HERE, s) for s in SOURCES]
 
 
+# The Python front end's bindings (csrc/fastcall.cpp): host code against this interpreter's and
+# this torch's headers, loaded by padra_amd/abi.py.  It links neither libpadra_hip.so nor the HIP
+# runtime: the library's functions are bound when it is loaded.
+FAST_SRC = os.path.join(HERE, "csrc", "fastcall.cpp")
+FAST_OUT = os.path.join(HERE, "_fastcall.so")
+
+
+def fast_command(out: str = FAST_OUT) -> list[str]:
+    import sysconfig
+
+    import torch
+    base = os.path.dirname(torch.__file__)
+    return ["g++", "-std=c++17", "-O2", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__=1",
+            "-DUSE_ROCM=1", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+            "-isystem", os.path.join(base, "include"),
+            "-isystem", os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "include"),
+            "-isystem", sysconfig.get_paths()["include"], "-I", os.path.join(ROOT, "include"),
+            "-o", out, FAST_SRC, "-L", os.path.join(base, "lib"), "-ltorch_python", "-ltorch_cpu",
+            "-lc10", "-lc10_hip"]
+
+
+def build_fast(out: str = FAST_OUT) -> str:
+    res = subprocess.run(fast_command(out), capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError("g++ failed (Python bindings):\n" + res.stdout + res.stderr)
+    return out
+
+
 CALLER_SRC = os.path.join(ROOT, "tests", "cpp", "padra_caller.cpp")
 CALLER_OUT = os.path.join(ROOT, "tests", "cpp", "padra_caller")
 
@@ -81,4 +109,5 @@ def build(out: str = OUT, verbose: bool = False, asan: bool = False) -> str:
 if __name__ == "__main__":
     print(build(verbose=True, asan="--asan" in sys.argv[1:]))
     if "--asan" not in sys.argv[1:]:
+        print(build_fast())
         print(build_caller())

@@ -14,29 +14,31 @@ import torch
 
 from . import abi
 
-_BF16_DTYPES = (torch.bfloat16, torch.int16, torch.uint16)
+_ACT = {torch.bfloat16: abi.ACT_BF16, torch.int16: abi.ACT_BF16, torch.uint16: abi.ACT_BF16,
+        torch.float32: abi.ACT_F32}
 
 
 def _act(t: torch.Tensor) -> int:
-    if t.dtype in _BF16_DTYPES:
-        return abi.ACT_BF16
-    if t.dtype == torch.float32:
-        return abi.ACT_F32
-    raise TypeError(f"activation dtype {t.dtype} (want bfloat16 or float32)")
-
-
-def _p(t):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
-
-
-def _stream(t: torch.Tensor):
-    return ctypes.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
-
-
-def _need_cuda(*ts):
-    for t in ts:
-        if t is not None and not t.is_cuda:
+    act = _ACT.get(t.dtype)
+    if act is None:
+        if not t.is_cuda:
             raise ValueError("padra_amd ops take GPU tensors")
+        raise TypeError(f"activation dtype {t.dtype} (want bfloat16 or float32)")
+    return act
+
+
+class _Calls:
+    """The entry points as csrc/fastcall.cpp binds them, on first use: each takes the tensor
+    whose device and current stream it runs on, then the C-ABI's arguments after `stream`
+    (tensors or None for device pointers).  A tensor that is not on the GPU raises ValueError,
+    a nonzero status PadraError."""
+
+    def __getattr__(self, name):
+        self.__dict__.update(abi.fast())
+        return self.__dict__[name]
+
+
+_c = _Calls()
 
 
 def ResidualPostNorm(x, residual, normalized, gamma, bad, eps=1e-6, tree=abi.TREE_128,
@@ -46,55 +48,48 @@ def ResidualPostNorm(x, residual, normalized, gamma, bad, eps=1e-6, tree=abi.TRE
     Replaces ResidualPostNormWideExact (tree=256), Add+Norm (tree=128)
     (residual_norm_wide_exact.cuh:6-80, inference.cu:188-214, 475-481).
     """
-    _need_cuda(x, residual, normalized, gamma, bad, statistics)
     rows, hidden = x.shape[0], x.shape[-1]
-    abi.call("padra_ResidualPostNorm", _stream(x), _p(x), _p(residual), _p(normalized),
-             _p(gamma), rows, hidden, float(eps), int(tree), _p(statistics), _p(bad), _act(x))
+    _c.padra_ResidualPostNorm(x, x, residual, normalized, gamma, rows, hidden, float(eps),
+                              int(tree), statistics, bad, _act(x))
 
 
 def NormFP8(x, normalized, gamma, packed, scales, bad, eps=1e-6, statistics=None):
     """normalized <- 128-thread RMSNorm of x; packed <- E4M3 codes of normalized/scale,
     scales[row] = max|normalized|/448 (NormFP8Exact, norm_fp8_exact.cuh:6-62)."""
-    _need_cuda(x, normalized, gamma, packed, scales, bad, statistics)
     rows, hidden = x.shape[0], x.shape[-1]
-    abi.call("padra_NormFP8", _stream(x), _p(x), _p(normalized), _p(gamma), _p(packed),
-             _p(scales), rows, hidden, float(eps), _p(statistics), _p(bad), _act(x))
+    _c.padra_NormFP8(x, x, normalized, gamma, packed, scales, rows, hidden, float(eps), statistics,
+                     bad, _act(x))
 
 
 def QuantizeFP8(x, packed, scales, bad):
     """packed <- E4M3 codes of x/scale, scales[row] = max|x|/448 (QuantizeFP8,
     prefill.cuh:46-66)."""
-    _need_cuda(x, packed, scales, bad)
-    abi.call("padra_QuantizeFP8", _stream(x), _p(x), _p(packed), _p(scales), x.shape[0],
-             x.shape[-1], _p(bad), _act(x))
+    _c.padra_QuantizeFP8(x, x, packed, scales, x.shape[0], x.shape[-1], bad, _act(x))
 
 
 def Combine(x, down, weights, bad, residual=True):
     """x <- [B(x + c) | c], c the ordered BF16 combine of the 8 expert rows
     (Combine, inference.cu:580-590).  down [rows][8][hidden], weights [rows][8] fp32."""
-    _need_cuda(x, down, weights, bad)
     rows, hidden = x.shape[0], x.shape[-1]
-    abi.call("padra_Combine", _stream(x), _p(x), _p(down), _p(weights), rows, hidden,
-             down.shape[1], int(bool(residual)), _p(bad), _act(x))
+    _c.padra_Combine(x, x, down, weights, rows, hidden, down.shape[1], int(bool(residual)), bad,
+                     _act(x))
 
 
 def CombineNorm(x, down, weights, normalized, gamma, bad, packed=None, scales=None, eps=1e-6,
                 statistics=None):
     """Residual combine, then RMSNorm (+ FP8 when packed is given)
     (combine_norm_exact::CombineNorm, combine_norm_exact.cuh:7-72)."""
-    _need_cuda(x, down, weights, normalized, gamma, bad, packed, scales, statistics)
     rows, hidden = x.shape[0], x.shape[-1]
-    abi.call("padra_CombineNorm", _stream(x), _p(x), _p(down), _p(weights), _p(normalized),
-             _p(gamma), _p(packed), _p(scales), rows, hidden, down.shape[1], float(eps),
-             _p(statistics), _p(bad), _act(x))
+    _c.padra_CombineNorm(x, x, down, weights, normalized, gamma, packed, scales, rows, hidden,
+                         down.shape[1], float(eps), statistics, bad, _act(x))
 
 
 def RopeTable(positions, head_dim=128, theta=1e6, yarn=False, factor=16.0,
               original_context=8192) -> torch.Tensor:
     """Host BF16 cos|sin table [positions][head_dim] (RopeTable, inference.cu:764-785)."""
     out = torch.empty((positions, head_dim), dtype=torch.int16)
-    abi.call("padra_RopeTable", _p(out), int(positions), int(head_dim), float(theta),
-             int(bool(yarn)), float(factor), int(original_context))
+    abi.call("padra_RopeTable", ctypes.c_void_p(out.data_ptr()), int(positions), int(head_dim),
+             float(theta), int(bool(yarn)), float(factor), int(original_context))
     return out.view(torch.bfloat16)
 
 
@@ -164,11 +159,9 @@ def QKNormRopeStore(q, k, qn, kn, table, positions: abi.Positions, bad, eps=1e-6
     Replaces QKNormRope / QKNormRopePair64 / QKNormRopeControlled /
     QKNormRopeStoreControlled and the cache writers after them (see padra_hip.h).
     """
-    _need_cuda(q, k, v, qn, kn, table, bad)
     tokens, q_heads, kv_heads, head_dim = _shape_qk(q, k)
-    abi.call("padra_QKNormRopeStore", _stream(q), _p(q), _p(k), _p(v), _p(qn), _p(kn),
-             _p(table), table.shape[0], ctypes.byref(positions), tokens, q_heads, kv_heads,
-             head_dim, float(eps), None if kv is None else ctypes.byref(kv), _p(bad), _act(q))
+    _c.padra_QKNormRopeStore(q, q, k, v, qn, kn, table, table.shape[0], positions, tokens, q_heads,
+                             kv_heads, head_dim, float(eps), kv, bad, _act(q))
 
 
 def ResidualNormQKRopeStore(x, residual, normalized, gamma, q, k, v, qn, kn, table,
@@ -176,70 +169,57 @@ def ResidualNormQKRopeStore(x, residual, normalized, gamma, q, k, v, qn, kn, tab
                             tree=abi.TREE_128, statistics=None):
     """ResidualPostNorm and QKNormRopeStore over the same tokens in one launch (BF16 or
     fp32 activations, by x's dtype)."""
-    _need_cuda(x, residual, normalized, gamma, q, k, v, qn, kn, table, bad, statistics)
     tokens, q_heads, kv_heads, head_dim = _shape_qk(q, k)
     if x.shape[0] != tokens:
         raise ValueError("x rows must equal the token count")
-    abi.call("padra_ResidualNormQKRopeStore", _stream(x), _p(x), _p(residual), _p(normalized),
-             _p(gamma), x.shape[-1], int(tree), _p(statistics), _p(q), _p(k), _p(v), _p(qn),
-             _p(kn), _p(table), table.shape[0], ctypes.byref(positions), tokens, q_heads,
-             kv_heads, head_dim, float(eps), None if kv is None else ctypes.byref(kv), _p(bad),
-             _act(x))
+    _c.padra_ResidualNormQKRopeStore(x, x, residual, normalized, gamma, x.shape[-1], int(tree),
+                                     statistics, q, k, v, qn, kn, table, table.shape[0], positions,
+                                     tokens, q_heads, kv_heads, head_dim, float(eps), kv, bad,
+                                     _act(x))
 
 
 def EmbedResidualNormQKRopeStore(embed, ids, x, residual, normalized, gamma, q, k, v, qn, kn,
                                  table, positions: abi.Positions, kv: abi.KVCache | None, bad,
                                  eps=1e-6, tree=abi.TREE_256, statistics=None):
     """Embed (x <- embed[token]) then ResidualNormQKRopeStore, in one launch."""
-    _need_cuda(embed, ids, x, residual, normalized, gamma, q, k, v, qn, kn, table, bad, statistics)
     tokens, q_heads, kv_heads, head_dim = _shape_qk(q, k)
     if x.shape[0] != tokens or embed.shape[-1] != x.shape[-1]:
         raise ValueError("x rows must equal the token count and embed rows x's width")
-    abi.call("padra_EmbedResidualNormQKRopeStore", _stream(x), _p(embed), embed.shape[0],
-             _p(ids), _p(x), _p(residual), _p(normalized), _p(gamma), x.shape[-1], int(tree),
-             _p(statistics), _p(q), _p(k), _p(v), _p(qn), _p(kn), _p(table), table.shape[0],
-             ctypes.byref(positions), tokens, q_heads, kv_heads, head_dim, float(eps),
-             None if kv is None else ctypes.byref(kv), _p(bad))
+    _c.padra_EmbedResidualNormQKRopeStore(x, embed, embed.shape[0], ids, x, residual, normalized,
+                                          gamma, x.shape[-1], int(tree), statistics, q, k, v, qn,
+                                          kn, table, table.shape[0], positions, tokens, q_heads,
+                                          kv_heads, head_dim, float(eps), kv, bad)
 
 
 def KVStore(k, v, positions: abi.Positions, kv: abi.KVCache, bad):
     """Store / encode K [T][Hkv][D] (already rotated) and V rows into the cache."""
-    _need_cuda(k, v, bad)
     tokens, kv_heads, head_dim = k.shape
-    abi.call("padra_KVStore", _stream(k), _p(k), _p(v), ctypes.byref(positions), tokens,
-             kv_heads, head_dim, ctypes.byref(kv), _p(bad), _act(k))
+    _c.padra_KVStore(k, k, v, positions, tokens, kv_heads, head_dim, kv, bad, _act(k))
 
 
 def KVCommit(chunk: abi.KVCache, ring: abi.KVCache, positions: abi.Positions, tokens, kv_heads,
              bad):
     """Copy encoded chunk rows r >= ring.first to ring slots position(r) % ring.cap."""
-    _need_cuda(bad)
-    abi.call("padra_KVCommit", _stream(bad), ctypes.byref(chunk), ctypes.byref(ring),
-             ctypes.byref(positions), int(tokens), int(kv_heads), _p(bad))
+    _c.padra_KVCommit(bad, chunk, ring, positions, int(tokens), int(kv_heads), bad)
 
 
 def KvQ8_0Dequantize(rows_k, rows_v, out_k, out_v, bad, kv_heads=4):
-    _need_cuda(rows_k, rows_v, out_k, out_v, bad)
-    abi.call("padra_KvQ8_0Dequantize", _stream(out_k), _p(rows_k), _p(rows_v), _p(out_k),
-             _p(out_v), rows_k.shape[0], int(kv_heads), _p(bad), _act(out_k))
+    _c.padra_KvQ8_0Dequantize(out_k, rows_k, rows_v, out_k, out_v, rows_k.shape[0], int(kv_heads),
+                              bad, _act(out_k))
 
 
 def KvQ8_0DequantizePrefix(rows_k, rows_v, out_k, out_v, positions: abi.Positions, tokens, bad,
                            kv_heads=4):
     """Decode the ring's first min(base, cap) rows (cap = rows_k.shape[0]) to BF16."""
-    _need_cuda(rows_k, rows_v, out_k, out_v, bad)
-    abi.call("padra_KvQ8_0DequantizePrefix", _stream(out_k), _p(rows_k), _p(rows_v), _p(out_k),
-             _p(out_v), ctypes.byref(positions), int(tokens), rows_k.shape[0], int(kv_heads),
-             _p(bad))
+    _c.padra_KvQ8_0DequantizePrefix(out_k, rows_k, rows_v, out_k, out_v, positions, int(tokens),
+                                    rows_k.shape[0], int(kv_heads), bad)
 
 
 def KVCheckpointCapture(ring: abi.KVCache, chunk: abi.KVCache, saved: abi.KVCache,
                         positions: abi.Positions, tokens, anchor, bad, kv_heads=4):
     """Snapshot of a 1024-row local ring at `anchor` (kv_checkpoint.cuh:27-89)."""
-    _need_cuda(bad)
-    abi.call("padra_KVCheckpointCapture", _stream(bad), ctypes.byref(ring), ctypes.byref(chunk),
-             ctypes.byref(saved), ctypes.byref(positions), int(tokens), int(anchor),
-             int(kv_heads), _p(bad))
+    _c.padra_KVCheckpointCapture(bad, ring, chunk, saved, positions, int(tokens), int(anchor),
+                                 int(kv_heads), bad)
 
 
 def DecodeAttention(q, kv: abi.KVCache, out, positions: abi.Positions, bad, kv_heads=4,
@@ -252,51 +232,41 @@ def DecodeAttention(q, kv: abi.KVCache, out, positions: abi.Positions, bad, kv_h
     raises ValueError.  Allocates the fp32 scratch when none is given.  With packed
     ([seqs][q_heads * 128] uint8) and scales ([seqs] fp32), the merge also writes each
     output row's E4M3 encoding (MergeQuantize, attention_merge_quantize_wide_exact.cuh:9-66)."""
-    _need_cuda(q, out, bad, scratch)
     seqs, q_heads = q.shape[0], q.shape[1]
-    used = abi.lib().padra_DecodeAttentionSplits(ctypes.byref(kv), seqs, int(kv_heads),
-                                                 int(bool(local)), int(splits))
+    used = _c.padra_DecodeAttentionSplits(kv, seqs, int(kv_heads), int(bool(local)),
+                                          int(splits))
     if used < 1:
         raise ValueError("invalid decode attention arguments")
-    need = abi.lib().padra_DecodeAttentionScratch(kv.format, seqs, q_heads, used)
+    need = _c.padra_DecodeAttentionScratch(kv.format, seqs, q_heads, used)
     if scratch is None:
         scratch = torch.empty(need, dtype=torch.float32, device=q.device)
     if packed is None:
-        abi.call("padra_DecodeAttention", _stream(q), _p(q), ctypes.byref(kv), _p(out),
-                 ctypes.byref(positions), seqs, q_heads, int(kv_heads), int(bool(local)),
-                 int(splits), _p(scratch), scratch.numel(), _p(bad), _act(q))
+        _c.padra_DecodeAttention(q, q, kv, out, positions, seqs, q_heads, int(kv_heads),
+                                 int(bool(local)), int(splits), scratch, scratch.numel(), bad,
+                                 _act(q))
     else:
-        _need_cuda(packed, scales)
-        abi.call("padra_DecodeAttentionFP8", _stream(q), _p(q), ctypes.byref(kv), _p(out),
-                 _p(packed), _p(scales), ctypes.byref(positions), seqs, q_heads, int(kv_heads),
-                 int(bool(local)), int(splits), _p(scratch), scratch.numel(), _p(bad), _act(q))
+        _c.padra_DecodeAttentionFP8(q, q, kv, out, packed, scales, positions, seqs, q_heads,
+                                    int(kv_heads), int(bool(local)), int(splits), scratch,
+                                    scratch.numel(), bad, _act(q))
     return scratch
 
 
 def RotateRows(data, bad, value=False):
     """In-place Hadamard rotation of 128-wide rows (K transform, or V with value=True)."""
-    _need_cuda(data, bad)
-    abi.call("padra_RotateRows", _stream(data), _p(data), data.numel() // 128, int(bool(value)),
-             _p(bad), _act(data))
+    _c.padra_RotateRows(data, data, data.numel() // 128, int(bool(value)), bad, _act(data))
 
 
 def SiluTableBuild(table):
     """table: device int16/uint16 [65536]."""
-    _need_cuda(table)
-    abi.call("padra_SiluTableBuild", _stream(table), _p(table))
+    _c.padra_SiluTableBuild(table, table)
 
 
 def SwiGLU(gate, up, out, table, bad):
-    _need_cuda(gate, up, out, table, bad)
-    abi.call("padra_SwiGLU", _stream(gate), _p(gate), _p(up), _p(out), gate.numel(), _p(table),
-             _p(bad), _act(gate))
+    _c.padra_SwiGLU(gate, gate, up, out, gate.numel(), table, bad, _act(gate))
 
 
 def Embed(table, out, bad, ids=None, positions: abi.Positions | None = None, tokens=None):
     """out[t] = table[token_t]; token from ids, a PrefillState prompt or DecodeStates."""
-    _need_cuda(table, out, bad, ids)
     vocab, hidden = table.shape
     tokens = out.shape[0] if tokens is None else tokens
-    abi.call("padra_Embed", _stream(out), _p(table), vocab, hidden, _p(ids),
-             None if positions is None else ctypes.byref(positions), int(tokens), _p(out),
-             _p(bad), _act(out))
+    _c.padra_Embed(out, table, vocab, hidden, ids, positions, int(tokens), out, bad, _act(out))
