@@ -904,21 +904,26 @@ __device__ __forceinline__ void bf16_split2(float x0, float x1, uint32_t &hi, ui
 }
 
 template <int G> __global__ __launch_bounds__(256) void k_q8_0_mx(AttnArgs a) {
-  // The 4 KV heads of a row, one wave each: the slice's rows are staged together, whole.
-  // K codes of the slice (rows padded to 36 words) and V codes as BF16 (4 keys per dimension
-  // and group, at slot vq_slot<true>(d)); head strides padded to 32 words modulo the banks.
-  __shared__ __align__(16) struct { uint32_t r[32][36]; uint32_t pad[32]; } kq_all[4];
-  __shared__ __align__(16) struct { uint2 r[8][kD + 8]; uint2 pad[16]; } vq_all[4];
-  __shared__ float ksc_all[4][32][4];    // K block scales by key
-  __shared__ float vsc_all[4][4][32];    // V block scales by block
-  __shared__ float ps_all[4][8][36];     // probabilities by head (rows padded)
+  // The 4 KV heads of a row, one wave each: the slice's rows are staged together, whole.  Per
+  // head: K codes (32 keys of 8 chunks, chunk c of a key at c ^ (key / 2) % 8), whose space the
+  // probabilities take once the wave has its scores; V codes as BF16 (4 keys per dimension and
+  // group j, at slot vq_slot<true>(d) ^ 16 ((j ^ j / 2) % 2)); block scales, K's as stored.  The
+  // exchanges and the heads' odd half-strides keep every access off the others' banks.
+  // Two barriers a slice and 53 KB, where a place of their own for the probabilities and a third
+  // barrier took 63 KB: 64 sequences of 8000 keys (32 heads) 98.4-100.5 -> 96.9-97.8 us, of 32768
+  // keys (16 heads) 246.6 -> 244.4.  The registers allow two workgroups a compute unit (218 VGPRs);
+  // held to three (168), the spills took twice the time.
+  __shared__ __align__(16) uint4 kq_all[4][256 + 8];
+  __shared__ __align__(16) uint2 vq_all[4][8 * kD + 16];
+  __shared__ __align__(8) uint2 ksc_all[4][32];        // K block scales (4 fp16) by key
+  __shared__ __align__(16) float vsc_all[4][4][32];    // V block scales by block
   const int tid = threadIdx.x, kv = tid >> 6;
   const int lane = tid & 63, col = lane & 15, grp = lane >> 4;
-  auto &kq = kq_all[kv].r;
-  auto &vq = vq_all[kv].r;
+  auto &kq = kq_all[kv];
+  auto &vq = vq_all[kv];
   auto &ksc = ksc_all[kv];
   auto &vsc = vsc_all[kv];
-  auto &ps = ps_all[kv];
+  float(&ps)[8][36] = *reinterpret_cast<float(*)[8][36]>(&kq_all[kv][0]); // by head (rows padded)
   AttnUnit unit;
   if (!attn_find<kQ8Tile>(a, tid == 0, unit))
     return; // block-uniform
@@ -1037,27 +1042,30 @@ template <int G> __global__ __launch_bounds__(256) void k_q8_0_mx(AttnArgs a) {
       }
 #pragma unroll
       for (int m = 0; m < 4; ++m) {
-        const int c = tid + 256 * m;
-        *reinterpret_cast<uint4 *>(&kq_all[(c >> 3) & 3].r[c >> 5][4 * (c & 7)]) = kw[m];
+        const int key = (tid >> 5) + 8 * m;
+        kq_all[(tid >> 3) & 3][8 * key + ((tid & 7) ^ ((key >> 1) & 7))] = kw[m];
       }
       {
-        float f[4][16];
+        const int t7 = tid & 7, j = tid >> 5;
+        uint2 *dst = &vq_all[(tid >> 3) & 3][j * kD + ((16 * t7) ^ (((j ^ (j >> 1)) & 1) << 4))];
+        // four dimensions at a time: without the scheduling barriers 251 VGPRs
 #pragma unroll
-        for (int m = 0; m < 4; ++m) {
-          const uint32_t w[4] = {vw[m].x, vw[m].y, vw[m].z, vw[m].w};
+        for (int i = 0; i < 4; ++i) {
+          float f[4][4];
 #pragma unroll
-          for (int i = 0; i < 4; ++i)
+          for (int m = 0; m < 4; ++m) {
+            const uint32_t w = i == 0 ? vw[m].x : i == 1 ? vw[m].y : i == 2 ? vw[m].z : vw[m].w;
 #pragma unroll
             for (int b = 0; b < 4; ++b)
-              f[m][4 * i + b] = (float)(int8_t)((w[i] >> (8 * b)) & 0xffu);
-        }
-        const int t7 = tid & 7;
-        uint2 *dst = &vq_all[(tid >> 3) & 3].r[tid >> 5][16 * t7];
+              f[m][b] = (float)(int8_t)((w >> (8 * b)) & 0xffu);
+          }
 #pragma unroll
-        for (int e = 0; e < 16; e += 2)
-          *reinterpret_cast<uint4 *>(dst + 2 * ((e / 2 + t7) & 7)) =
-              make_uint4(pack2(f[0][e], f[1][e]), pack2(f[2][e], f[3][e]),
-                         pack2(f[0][e + 1], f[1][e + 1]), pack2(f[2][e + 1], f[3][e + 1]));
+          for (int e = 0; e < 4; e += 2)
+            *reinterpret_cast<uint4 *>(dst + 2 * ((2 * i + e / 2 + t7) & 7)) =
+                make_uint4(pack2(f[0][e], f[1][e]), pack2(f[2][e], f[3][e]),
+                           pack2(f[0][e + 1], f[1][e + 1]), pack2(f[2][e + 1], f[3][e + 1]));
+          __builtin_amdgcn_sched_barrier(0);
+        }
       }
       if (tid < 128) {
         const bool inside = o0 + hrow < n;
@@ -1065,19 +1073,14 @@ template <int G> __global__ __launch_bounds__(256) void k_q8_0_mx(AttnArgs a) {
 #pragma unroll
         for (int h2 = 0; h2 < 2; ++h2) { // heads 2 (tid % 2) + h2
           const int hd = 2 * (tid & 1) + h2;
-          float d[4];
-#pragma unroll
-          for (int b = 0; b < 4; ++b) {
-            const uint32_t word = hv[2 * h2 + (b >> 1)];
-            d[b] = inside ? f16_bits((b & 1) ? word >> 16 : word & 0xffffu) : 0.f;
-          }
+          const uint32_t w0 = inside ? hv[2 * h2] : 0u, w1 = inside ? hv[2 * h2 + 1] : 0u;
           if (tid < 64) {
-            *reinterpret_cast<float4 *>(&ksc_all[hd][hrow][0]) =
-                make_float4(d[0], d[1], d[2], d[3]);
+            ksc_all[hd][hrow] = make_uint2(w0, w1);
           } else {
-#pragma unroll
-            for (int b = 0; b < 4; ++b)
-              vsc_all[hd][b][hrow] = d[b];
+            vsc_all[hd][0][hrow] = f16_bits(w0 & 0xffffu);
+            vsc_all[hd][1][hrow] = f16_bits(w0 >> 16);
+            vsc_all[hd][2][hrow] = f16_bits(w1 & 0xffffu);
+            vsc_all[hd][3][hrow] = f16_bits(w1 >> 16);
           }
         }
       }
@@ -1094,9 +1097,11 @@ template <int G> __global__ __launch_bounds__(256) void k_q8_0_mx(AttnArgs a) {
       float sc[2][2];
 #pragma unroll
       for (int k = 0; k < 2; ++k) {
-        const uint4 b0 = *reinterpret_cast<const uint4 *>(&kq[16 * k + col][4 * grp]);
-        const uint4 b1 = *reinterpret_cast<const uint4 *>(&kq[16 * k + col][16 + 4 * grp]);
-        const float4 kd = *reinterpret_cast<const float4 *>(&ksc[16 * k + col][0]);
+        const uint4 b0 = kq[8 * (16 * k + col) + (grp ^ (col >> 1))];
+        const uint4 b1 = kq[8 * (16 * k + col) + ((4 + grp) ^ (col >> 1))];
+        const uint2 kh = ksc[16 * k + col];
+        const float4 kd = make_float4(f16_bits(kh.x & 0xffffu), f16_bits(kh.x >> 16),
+                                      f16_bits(kh.y & 0xffffu), f16_bits(kh.y >> 16));
         const bool valid = o0 + 16 * k + col < n;
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
@@ -1136,7 +1141,7 @@ template <int G> __global__ __launch_bounds__(256) void k_q8_0_mx(AttnArgs a) {
             o[t][i] *= ar;
         }
       }
-      __syncthreads();
+      // (The probabilities are the wave's own: its LDS accesses run in program order.)
       // PV A operands: row col = (head col % 8, block 2 c + col / 8); K-slots of group grp are
       // keys 8 grp .. 8 grp + 7.
       uint4 ahi[2], alo[2];
@@ -1164,8 +1169,8 @@ template <int G> __global__ __launch_bounds__(256) void k_q8_0_mx(AttnArgs a) {
       }
 #pragma unroll
       for (int t = 0; t < 8; ++t) {
-        const int d = vq_slot<true>(16 * t + col);
-        const uint2 v0 = vq[2 * grp][d], v1 = vq[2 * grp + 1][d];
+        const int d = vq_slot<true>(16 * t + col) ^ ((grp & 1) << 4);
+        const uint2 v0 = vq[2 * grp * kD + d], v1 = vq[(2 * grp + 1) * kD + (d ^ 16)];
         const uint4 bv = make_uint4(v0.x, v0.y, v1.x, v1.y);
         o[t] = mfma_bf16(ahi[t >> 2], bv, o[t]);
         o[t] = mfma_bf16(alo[t >> 2], bv, o[t]);
