@@ -48,6 +48,81 @@ __device__ __forceinline__ float silu_entry(uint32_t gb, const uint16_t *lut) {
   return __uint_as_float((uint32_t)lut[sign * kLutSpan + (mag - kLutLo)] << 16);
 }
 
+// Eight elements at p + at: consecutive (BF16), or four at `at` and four 256 further (fp32).
+__device__ __forceinline__ void load8_pieces(const uint16_t *p, long long at, bool in, bool,
+                                             float other, float (&v)[8]) {
+#pragma unroll
+  for (int k = 0; k < 8; ++k)
+    v[k] = other;
+  if (in)
+    ActIO<uint16_t>::load8(p + at, v);
+}
+__device__ __forceinline__ void load8_pieces(const float *p, long long at, bool in0, bool in1,
+                                             float other, float (&v)[8]) {
+  const uint32_t o = __float_as_uint(other);
+  uint4 a = make_uint4(o, o, o, o), b = a;
+  if (in0)
+    a = ld_nt(reinterpret_cast<const uint4 *>(p + at));
+  if (in1)
+    b = ld_nt(reinterpret_cast<const uint4 *>(p + at + 256));
+  const uint32_t w[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+#pragma unroll
+  for (int k = 0; k < 8; ++k)
+    v[k] = __uint_as_float(w[k]);
+}
+__device__ __forceinline__ void store8_pieces(uint16_t *p, long long at, bool in, bool,
+                                              const uint32_t (&w)[4]) {
+  if (in)
+    ActIO<uint16_t>::store8(p + at, w);
+}
+__device__ __forceinline__ void store8_pieces(float *p, long long at, bool in0, bool in1,
+                                              const uint32_t (&w)[4]) {
+  if (in0)
+    st_nt(reinterpret_cast<uint4 *>(p + at),
+          make_uint4(w[0] << 16, w[0] & 0xffff0000u, w[1] << 16, w[1] & 0xffff0000u));
+  if (in1)
+    st_nt(reinterpret_cast<uint4 *>(p + at + 256),
+          make_uint4(w[2] << 16, w[2] & 0xffff0000u, w[3] << 16, w[3] & 0xffff0000u));
+}
+
+// Eight elements whose gates are BF16-exact with a table entry in the span and whose ups are
+// finite, which the caller has established for the whole wave: the look-up and the product without
+// a branch.  gp: the gates' BF16 pairs.
+__device__ __forceinline__ void swiglu8(const uint32_t (&gp)[4], const float (&u)[8],
+                                        const uint16_t *lut, uint32_t (&w)[4], bool &fine) {
+  float r[8];
+  uint32_t s[8];
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    const uint32_t gb = (k & 1) ? gp[k / 2] >> 16 : gp[k / 2];
+    const uint32_t mag = gb & 0x7fffu, sign = (gb >> 15) & 1u;
+    s[k] = lut[sign * kLutSpan + (mag - kLutLo)];
+  }
+  float most = 0.f;
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    r[k] = __uint_as_float(s[k] << 16) * u[k]; // finite operands: no NaN for fmaxf to drop
+    most = fmaxf(most, fabsf(r[k]));
+  }
+  fine = fine && bf16_finite(most);
+#pragma unroll
+  for (int p = 0; p < 4; ++p)
+    w[p] = pack2(r[2 * p], r[2 * p + 1]);
+}
+
+// Whether every gate of four BF16 pairs has a table entry in the span.
+__device__ __forceinline__ bool in_span(const uint32_t (&gp)[4]) {
+  typedef uint16_t u16x2_t __attribute__((ext_vector_type(2)));
+  u16x2_t lo = __builtin_bit_cast(u16x2_t, gp[0] & 0x7fff7fffu), hi = lo;
+#pragma unroll
+  for (int p = 1; p < 4; ++p) {
+    const u16x2_t m = __builtin_bit_cast(u16x2_t, gp[p] & 0x7fff7fffu);
+    lo = __builtin_elementwise_min(lo, m);
+    hi = __builtin_elementwise_max(hi, m);
+  }
+  return min((uint32_t)lo.x, (uint32_t)lo.y) >= kLutLo && max((uint32_t)hi.x, (uint32_t)hi.y) < kLutHi;
+}
+
 // exl3_silu_lut::Activate (exl3_silu_lut.cuh:15-31): out = B(s * up), s the table entry of
 // the gate.  A non-finite gate or up raises the flag and leaves the gate value in `out`
 // (the reference skips the element of its in-place output); a non-finite product raises
@@ -64,12 +139,37 @@ __global__ __launch_bounds__(512) void k_swiglu(const T *gate, const T *up, T *o
   }
   __syncthreads();
   bool fine = true;
-  for (long long gi = blockIdx.x * (long long)blockDim.x + threadIdx.x; gi < groups;
-       gi += (long long)gridDim.x * blockDim.x) {
+  // Eight elements a lane: consecutive in BF16; in fp32 two fours, 256 elements apart in the
+  // wave's 512, so that each instruction covers whole lines: with lanes 32 bytes apart, as eight
+  // consecutive fp32 elements are, 16384 x 1024 took 52.2 us (3.9 TB/s), now 34.5 (5.8).
+  constexpr bool F32 = std::is_same<T, float>::value;
+  const int lane = threadIdx.x & 63;
+  for (long long wave = blockIdx.x * 8ll + (threadIdx.x >> 6); wave * 64 < groups;
+       wave += gridDim.x * 8ll) {
+    const long long at = wave * 512 + (F32 ? 4 : 8) * lane; // the lane's first element
+    const bool in0 = at < groups * 8, in1 = F32 ? at + 256 < groups * 8 : in0;
     float g[8], u[8];
-    ActIO<T>::load8(gate + gi * 8, g);
-    ActIO<T>::load8(up + gi * 8, u);
+    load8_pieces(gate, at, in0, in1, 1.f, g); // past the end: silu(1) * 0
+    load8_pieces(up, at, in0, in1, 0.f, u);
     uint32_t w[4];
+    // Ordinary data (nearly always): no element needs a closed form or raises the flag before its
+    // product, tested once for the wave's 512 elements.  With tests and branches for each element
+    // (below, now for the other waves) the arithmetic did not hide behind the memory:
+    // 16384 x 1024 BF16 20.8-21.5 -> 19.8 us, cold (5.1 TB/s), 512 x 896 4.4 -> 3.7, 8 x 896 4.0 -> 3.1.
+    uint32_t gp[4], inexact = 0, um = 0;
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+      const uint32_t g0 = __float_as_uint(g[2 * p]), g1 = __float_as_uint(g[2 * p + 1]);
+      gp[p] = __builtin_amdgcn_perm(g1, g0, 0x07060302u);
+      inexact |= g0 | g1;
+      um = max(um, max(__float_as_uint(u[2 * p]) & 0x7fffffffu,
+                       __float_as_uint(u[2 * p + 1]) & 0x7fffffffu));
+    }
+    if (__ballot(!in_span(gp) || (inexact & 0xffffu) != 0 || um >= 0x7f800000u) == 0) {
+      swiglu8(gp, u, lut, w, fine);
+      store8_pieces(out, at, in0, in1, w);
+      continue;
+    }
 #pragma unroll
     for (int p = 0; p < 4; ++p) {
       float r[2];
@@ -88,7 +188,7 @@ __global__ __launch_bounds__(512) void k_swiglu(const T *gate, const T *up, T *o
       }
       w[p] = pack2(r[0], r[1]);
     }
-    ActIO<T>::store8(out + gi * 8, w);
+    store8_pieces(out, at, in0, in1, w);
   }
   if (!fine)
     raise_bad(bad);
