@@ -29,10 +29,26 @@ int launched(const char *what) {
 }
 bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
-// The combine of 8 consecutive columns: every load (the row's 8 weights, the 8 expert rows,
+template <class T, int PIECE> __device__ __forceinline__ void load8_piece(const T *p, float (&v)[8]) {
+  if constexpr (PIECE == 4) {
+    ActIO<T>::load8(p, v);
+  } else {
+    const uint4 a = ld_nt(reinterpret_cast<const uint4 *>(p));
+    const uint4 b = ld_nt(reinterpret_cast<const uint4 *>(p + PIECE));
+    const uint32_t w[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+      v[k] = __uint_as_float(w[k]);
+  }
+}
+
+// The combine of 8 columns: every load (the row's 8 weights, the 8 expert rows,
 // x) is issued before the arithmetic.  Returns the packed BF16 results; `fine` is false
 // when one of them is not finite.
-template <class T, bool RES>
+// PIECE: distance of the lane's second four columns from its first four, 4 where the eight are
+// consecutive.  In fp32 the callers place them 256 apart, so that each instruction covers whole
+// lines: with lanes 32 bytes apart it touched every second 16 bytes of twice as many.
+template <class T, bool RES, int PIECE = 4>
 __device__ __forceinline__ void combine8(const T *x, const T *down, size_t expert_stride,
                                          const float *w, uint32_t (&out)[4], bool &fine) {
   float d[kExperts][8], xv[8];
@@ -42,9 +58,9 @@ __device__ __forceinline__ void combine8(const T *x, const T *down, size_t exper
     wt[e] = w[e];
 #pragma unroll
   for (int e = 0; e < kExperts; ++e)
-    ActIO<T>::load8(down + e * expert_stride, d[e]);
+    load8_piece<T, PIECE>(down + e * expert_stride, d[e]);
   if constexpr (RES)
-    ActIO<T>::load8(x, xv);
+    load8_piece<T, PIECE>(x, xv);
   float c[8];
 #pragma unroll
   for (int k = 0; k < 8; ++k)
@@ -115,19 +131,31 @@ __global__ __launch_bounds__(64 * W) void k_combine_norm(T *x, const T *down, co
   bool fine = true;
 #pragma unroll
   for (int i = 0; i < (CHUNKS + W - 1) / W; ++i) {
-    const int ch = wave + W * i, col = ch * 512 + 8 * lane;
-    if (ch < CHUNKS && col < H) {
+    // a chunk's lane: columns 4l .. 4l + 3 and the same of its second half; a last chunk of 256
+    // columns has 8l .. 8l + 7 of its lower lanes
+    const int ch = wave + W * i;
+    auto piece = [&](auto apart, int col) {
+      constexpr int P = decltype(apart)::value;
       T *xr = x + (size_t)row * H + col;
       uint32_t out[4];
       bool f;
-      combine8<T, true>(xr, down + (size_t)row * kExperts * H + col, (size_t)H,
-                        weights + (size_t)row * kExperts, out, f);
-      ActIO<T>::template store8<true>(xr, out);
+      combine8<T, true, P>(xr, down + (size_t)row * kExperts * H + col, (size_t)H,
+                           weights + (size_t)row * kExperts, out, f);
+      st_wt(reinterpret_cast<uint4 *>(xr), make_uint4(out[0] << 16, out[0] & 0xffff0000u,
+                                                      out[1] << 16, out[1] & 0xffff0000u));
+      st_wt(reinterpret_cast<uint4 *>(xr + P), make_uint4(out[2] << 16, out[2] & 0xffff0000u,
+                                                          out[3] << 16, out[3] & 0xffff0000u));
       fine = fine && f;
 #pragma unroll
-      for (int k = 0; k < 4; ++k)
+      for (int k = 0; k < 2; ++k) {
         v_lds[col / 2 + k] = out[k];
-    }
+        v_lds[(col + P) / 2 + k] = out[2 + k];
+      }
+    };
+    if (ch * 512 + 512 <= H)
+      piece(std::integral_constant<int, 256>{}, ch * 512 + 4 * lane);
+    else if (ch < CHUNKS && ch * 512 + 8 * lane < H)
+      piece(std::integral_constant<int, 4>{}, ch * 512 + 8 * lane);
   }
   if (__ballot(!fine) != 0 && lane == 0)
     raise_bad(a.bad);
