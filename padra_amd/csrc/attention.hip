@@ -339,8 +339,9 @@ __global__ __launch_bounds__(64 * W) void k_attn_mx(AttnArgs a) {
   constexpr int NB = 8 / W; // 16-dimension blocks of the output per wave
   const int G = a.group;
   // Per tile of the round: (V[4j][d], V[4j+1][d]), (V[4j+2][d], V[4j+3][d]) at slot
-  // vq_slot(d) ^ 16 (j % 2) (odd groups half the banks away from even ones); the probabilities in the A operand's layout; per query row, the tile's
-  // maximum, its rescale factor and its sum of probabilities.
+  // vq_slot(d) ^ 16 (j % 2) (odd groups half the banks away from even ones); the probabilities in
+  // the A operand's layout; per query row, the tile's maximum, its rescale factor and its sum of
+  // probabilities.
   __shared__ __align__(16) uint2 vq[W][kKeys / 4][kD];
   __shared__ __align__(16) uint4 pq[W][64];
   __shared__ __align__(16) float tile_max[W][16], tile_alpha[W][16], tile_total[W][16];
@@ -667,8 +668,9 @@ __global__ __launch_bounds__(64 * W) void k_attn_mx(AttnArgs a) {
 }
 
 // Partial outputs of one (sequence, head), a float2 per lane and split.  The merge kernels are
-// bound by their chain of memory round trips (control record, log-sum-exps, partials), so they issue every split's load before the first use and, in small launches,
-// before the control record is there: the splits that turn out inactive are read in vain,
+// bound by their chain of memory round trips (control record, log-sum-exps, partials), so they
+// issue every split's load before the first use and, in small launches, before the control record
+// is there: the splits that turn out inactive are read in vain,
 // inside the scratch.  Launches of more heads read only the active ones: there the bytes count.
 // Steps of 1 / 8 / 64 sequences (1000, 8000, 8000 keys), before -> after: BF16 10.3 -> 8.5,
 // 25.2 -> 23.8, 103.6 -> 104.2 us; q8_0 21.9 -> 20.3, 39.2 -> 31.6, 107.1 -> 102.6 us.
@@ -1243,8 +1245,9 @@ template <int G> __global__ __launch_bounds__(256) void k_q8_0_mx(AttnArgs a) {
 
 // ---- q8_0 split for few sequences -------------------------------------------------------
 // k_q8_0_mx walks the four streams of a split one after the other, with a workgroup per (sequence,
-// split) and a wave per KV head: one sequence ran 32 workgroups, 128 waves in all.  Here a workgroup takes one (sequence, split, KV head) and its four waves
-// one stream each, so that four times the waves walk a quarter of the slices, without a
+// split) and a wave per KV head: one sequence ran 32 workgroups, 128 waves in all.  Here a
+// workgroup takes one (sequence, split, KV head) and its four waves one stream each, so that four
+// times the waves walk a quarter of the slices, without a
 // barrier on the way; then each wave folds one row of every head's streams.  The query is
 // coded here too, while the first slice is on its way, which saves that launch.  Every sum has the
 // order it has in k_q8_0_mx: the bits are the same.
