@@ -615,8 +615,8 @@ int chain(hipStream_t s, const uint16_t *gather, int vocab, const int32_t *ids, 
 } // namespace
 
 namespace {
-// The chain on fp32 activations (the reference's buffers), in one launch: up to
-// head_wave_tokens of norm-row waves and per-head Q/K waves.
+// The chain on fp32 activations (the reference's buffers), in one launch but for one corner
+// (below): up to head_wave_tokens of norm-row waves and per-head Q/K waves.
 int chain_f32(hipStream_t s, void *x, const void *residual, void *normalized,
               const uint16_t *gamma, int hidden, int tree, float *statistics, void *q, void *k,
               const void *v, const uint16_t *qn, const uint16_t *kn, const uint16_t *table,
@@ -660,6 +660,20 @@ int chain_f32(hipStream_t s, void *x, const void *residual, void *normalized,
       //                         2048        22.8 : 22.7  24.1 : 25.4  25.0 : 26.5
       //   hidden 2304, 32 heads, 512 tokens 10.1 : 13.2  12.5 : 15.5  12.1 : 15.3
       //                         2048        30.2 : 33.4  31.4 : 34.7  31.7 : 35.0
+      // Only where few heads and no encoding leave the Q/K part short beside many norm rows do
+      // two kernels come out ahead (16 heads, BF16 cache: 1400 tokens 17.5 : 17.7, 2048 tokens 22.8 :
+      // 22.7 here and 22.2 : 21.3 with all inputs cold): from 1792 tokens of at most 20 heads.
+      if (fmt.value <= PADRA_KV_BF16 && tokens >= 1792 && q_heads + kv_heads <= 20) {
+        hipLaunchKernelGGL((k_norm<vt.value, j.value, float, true>), dim3((unsigned)norm_waves),
+                           dim3(64), 0, s, n);
+        const int st2 = launched();
+        if (st2)
+          return st2;
+        hipLaunchKernelGGL((k_qk<float, fmt.value>),
+                           dim3((unsigned)qk_wave_count<fmt.value>(tokens, q_heads, kv_heads)),
+                           dim3(64), 0, s, a);
+        return launched();
+      }
       const long long waves = norm_waves + qk_wave_count<fmt.value>(tokens, q_heads, kv_heads);
       hipLaunchKernelGGL((k_chain<vt.value, j.value, fmt.value, false, float>),
                          dim3((unsigned)waves), dim3(64), 0, s, n, a, norm_waves, waves);

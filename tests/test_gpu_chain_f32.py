@@ -21,7 +21,8 @@ def gpu():
 @pytest.mark.parametrize("tokens,hidden,heads,tree", [(321, 2048, 16, abi.TREE_128),
                                                       (385, 2304, 32, abi.TREE_256),
                                                       (1201, 2304, 32, abi.TREE_128),
-                                                      (2048, 2048, 4, abi.TREE_256)])
+                                                      (2048, 2048, 4, abi.TREE_256),
+                                                      (1793, 2048, 16, abi.TREE_128)])
 def test_chain_f32_equals_its_halves(fmt, tokens, hidden, heads, tree):
     """Just past the per-head sizes (320 tokens with a quantized cache, 384 without), odd chunk
     sizes, a local ring narrower than the chunk, a NaN row: every output and the flag equal."""
