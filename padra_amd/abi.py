@@ -151,7 +151,7 @@ def fast() -> dict:
         import torch  # noqa: F401  (the libraries that _fastcall.so links)
 
         from . import _fastcall
-        _fast = _fastcall.bind(library_path, PadraError)
+        _fast = _fastcall.bind(library_path, PadraError, Positions, KVCache)
     return _fast
 
 

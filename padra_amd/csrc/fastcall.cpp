@@ -1,6 +1,6 @@
 // The Python front end's way into libpadra_hip.so: one function per entry point, with the
 // C-ABI's arguments after the tensor whose device and current stream the call runs on.  A
-// device pointer is a tensor (or None), a descriptor its ctypes structure (or None).
+// device pointer is a tensor (or None), a descriptor its own ctypes structure (or None).
 //
 // A decode step's kernels take 3-5 us, and ctypes with its Python-side conversions took 8-16 us a
 // call, so the calls and not the kernels set the time of every small launch.  These read the
@@ -24,6 +24,8 @@ namespace {
 struct PythonError {}; // the interpreter's error indicator is set
 
 PyObject *g_error = nullptr; // abi.PadraError
+// The descriptors' ctypes structures, as abi.py declares them.
+template <class S> PyObject *g_structure = nullptr;
 
 const at::Tensor *tensor(PyObject *o) {
   return THPVariable_CheckExact(o) ? &THPVariable_Unpack(o) : nullptr;
@@ -85,19 +87,21 @@ void *stream_of(PyObject *o) {
   return c10::hip::getCurrentHIPStream(index).stream();
 }
 
+// A descriptor: its own ctypes structure (or a subclass) and nothing else.  A KVCache is large
+// enough for a Positions, and its plane pointers would be read as control records.
 template <class S> const S *descriptor(PyObject *o) {
   if (o == Py_None)
     return nullptr;
+  PyTypeObject *type = reinterpret_cast<PyTypeObject *>(g_structure<S>);
+  if (!PyObject_TypeCheck(o, type)) {
+    PyErr_Format(PyExc_TypeError, "expected %s, not %s", type->tp_name, Py_TYPE(o)->tp_name);
+    throw PythonError{};
+  }
   Py_buffer view;
   if (PyObject_GetBuffer(o, &view, PyBUF_SIMPLE) != 0)
     throw PythonError{};
   const S *s = static_cast<const S *>(view.buf);
-  const bool whole = view.len >= (Py_ssize_t)sizeof(S);
   PyBuffer_Release(&view); // the structure's memory lives as long as the caller's object
-  if (!whole) {
-    PyErr_SetString(PyExc_TypeError, "descriptor structure too small");
-    throw PythonError{};
-  }
   return s;
 }
 
@@ -127,22 +131,18 @@ template <class A> A argument(PyObject *o) {
   }
 }
 
-template <size_t I, bool LAUNCH, class A> A argument_at(PyObject *const *args) {
-  if constexpr (LAUNCH && I == 0)
-    return stream_of(args[0]);
-  else
-    return argument<A>(args[I]);
-}
-
 // One library function, bound at run time in the build that abi.library_path names.
 template <auto Declared> struct Entry;
 template <class R, class... A, R (*Declared)(A...)> struct Entry<Declared> {
   static inline R (*function)(A...) = nullptr;
   static inline const char *name = nullptr;
 
+  // (Every argument is checked, left to right, before torch is asked for the stream.)
   template <bool LAUNCH, size_t... I>
   static R run(PyObject *const *args, std::index_sequence<I...>) {
-    const std::tuple<A...> values{argument_at<I, LAUNCH, A>(args)...}; // left to right
+    std::tuple<A...> values{LAUNCH && I == 0 ? A{} : argument<A>(args[I])...};
+    if constexpr (LAUNCH)
+      std::get<0>(values) = stream_of(args[0]);
     PyThreadState *state = PyEval_SaveThread(); // as ctypes does: a launch may wait for room
     const R r = function(std::get<I>(values)...);
     PyEval_RestoreThread(state);
@@ -218,11 +218,26 @@ Listed g_listed[] = {
     VALUE(padra_DecodeAttentionScratch),
 };
 
-// bind(library path, PadraError) -> {entry point: function}
+// Whether o is a ctypes structure type of S's size.
+template <class S> bool is_structure(PyObject *o) {
+  PyObject *e = PyType_Check(o) ? PyObject_CallNoArgs(o) : nullptr;
+  Py_buffer view;
+  const bool same = e && PyObject_GetBuffer(e, &view, PyBUF_SIMPLE) == 0;
+  const bool whole = same && view.len == (Py_ssize_t)sizeof(S);
+  if (same)
+    PyBuffer_Release(&view);
+  Py_XDECREF(e);
+  if (!whole && !PyErr_Occurred())
+    PyErr_SetString(PyExc_TypeError, "bind takes the descriptors' ctypes structures");
+  return whole;
+}
+
+// bind(library path, PadraError, Positions, KVCache) -> {entry point: function}
 PyObject *bind(PyObject *, PyObject *args) {
   const char *path;
-  PyObject *error;
-  if (!PyArg_ParseTuple(args, "sO", &path, &error))
+  PyObject *error, *positions, *cache;
+  if (!PyArg_ParseTuple(args, "sOOO", &path, &error, &positions, &cache) ||
+      !is_structure<padra_Positions>(positions) || !is_structure<padra_KVCache>(cache))
     return nullptr;
   void *library = dlopen(path, RTLD_NOW | RTLD_LOCAL);
   if (!library) {
@@ -245,6 +260,10 @@ PyObject *bind(PyObject *, PyObject *args) {
   }
   Py_INCREF(error);
   Py_XSETREF(g_error, error);
+  Py_INCREF(positions);
+  Py_XSETREF(g_structure<padra_Positions>, positions);
+  Py_INCREF(cache);
+  Py_XSETREF(g_structure<padra_KVCache>, cache);
   return all;
 }
 

@@ -1,9 +1,29 @@
 """The tensor bindings of the entry points (csrc/fastcall.cpp): what they refuse, and the tensors
 and streams they take."""
+import ctypes
+
+import numpy as np
 import pytest
 import torch
 
 from padra_amd import abi, ops
+
+
+class _OnGpu:
+    """What a binding reads of a tensor, for calls that are refused before the library's."""
+    is_cuda, dtype = True, torch.bfloat16
+
+    def __init__(self, *shape):
+        self.shape = shape
+
+    def data_ptr(self):
+        return 4096
+
+    def get_device(self):
+        return 0
+
+    def numel(self):
+        return 1
 
 
 def test_cpu_tensors_are_refused():
@@ -26,8 +46,6 @@ def test_argument_errors():
         calls["padra_SwiGLU"](None)
     with pytest.raises(TypeError):  # a descriptor that is no structure
         calls["padra_DecodeAttentionSplits"](3, 1, 4, 0, 0)
-    with pytest.raises(TypeError, match="too small"):
-        calls["padra_DecodeAttentionSplits"](bytes(8), 1, 4, 0, 0)
     with pytest.raises(AttributeError):  # the stream's tensor
         calls["padra_SiluTableBuild"](None, None)
     kv = abi.KVCache(format=abi.KV_Q8_0, k=None, v=None, scales=None, cap=1024, first=0,
@@ -37,6 +55,36 @@ def test_argument_errors():
         assert calls["padra_DecodeAttentionSplits"](kv, *args) == lib.padra_DecodeAttentionSplits(kv, *args)
     assert calls["padra_DecodeAttentionScratch"](2, 1 << 16, 32, 32) == \
         lib.padra_DecodeAttentionScratch(2, 1 << 16, 32, 32) > 1 << 32
+
+
+def test_descriptors_are_their_own_structures():
+    """A structure of the other kind, or bytes of the right size, are refused before any call (a
+    KVCache is larger than a Positions: its words would be read as a mode and control records)."""
+    calls = abi.fast()
+    from padra_amd import _fastcall
+    kv = abi.KVCache(format=abi.KV_Q8_0, cap=1024)
+    size = ctypes.sizeof(kv)
+    assert size >= ctypes.sizeof(abi.Positions)
+    for wrong in (ops.positions_base(0), bytes(kv), bytearray(kv), np.zeros(size, np.uint8),
+                  (abi.KVCache * 2)(), ctypes.pointer(kv)):
+        with pytest.raises(TypeError, match="expected KVCache"):
+            calls["padra_DecodeAttentionSplits"](wrong, 1, 4, 0, 0)
+    x = _OnGpu()
+    for wrong in (kv, bytes(size)):
+        with pytest.raises(TypeError, match="expected Positions"):
+            calls["padra_Embed"](x, x, 8, 8, None, wrong, 1, x, x, 0)
+        with pytest.raises(TypeError, match="expected Positions"):
+            ops.DecodeAttention(_OnGpu(1, 8, 128), kv, x, wrong, x, scratch=x)
+
+    class Derived(abi.KVCache):
+        pass
+
+    derived = Derived(format=abi.KV_Q8_0, cap=1024)
+    assert calls["padra_DecodeAttentionSplits"](derived, 1, 4, 0, 0) == 32
+    for classes in ((abi.KVCache, abi.Positions), (abi.Positions, kv), (int, abi.KVCache)):
+        with pytest.raises(TypeError):
+            _fastcall.bind(abi.library_path, abi.PadraError, *classes)
+    assert calls["padra_DecodeAttentionSplits"](kv, 1, 4, 0, 0) == 32
 
 
 @pytest.mark.gpu
