@@ -5,8 +5,9 @@
 // A decode step's kernels take 3-5 us, and ctypes with its Python-side conversions took 8-16 us a
 // call, so the calls and not the kernels set the time of every small launch.  These read the
 // tensors themselves: a decode step's call 10.5 -> 5.0 us, the three calls of a chunk's ring work
-// 22.0 -> 12.3 us, its kernels' time.  The checks are those of the Python code
-// they replace: a tensor that is not on the GPU raises ValueError, a nonzero status PadraError.
+// 22.0 -> 12.3 us, its kernels' time.  The checks are those of the Python code and of ctypes that
+// they replace: a tensor that is not on the GPU raises ValueError, another structure than the
+// descriptor's or a count that is no integer TypeError, a nonzero status PadraError.
 #include <dlfcn.h>
 
 #include <c10/hip/HIPStream.h>
@@ -113,14 +114,12 @@ template <class A> A argument(PyObject *o) {
   } else if constexpr (std::is_pointer_v<A>) {
     return static_cast<A>(address(o));
   } else if constexpr (std::is_floating_point_v<A>) {
-    PyObject *f = PyNumber_Float(o);
-    if (!f)
+    const double v = PyFloat_AsDouble(o);
+    if (v == -1. && PyErr_Occurred())
       throw PythonError{};
-    const double v = PyFloat_AS_DOUBLE(f);
-    Py_DECREF(f);
     return (A)v;
   } else {
-    PyObject *i = PyNumber_Long(o);
+    PyObject *i = PyNumber_Index(o); // an integer, as ctypes asks: 1.9 or "2" is a TypeError
     if (!i)
       throw PythonError{};
     const unsigned long long v = PyLong_AsUnsignedLongLongMask(i);

@@ -87,6 +87,27 @@ def test_descriptors_are_their_own_structures():
     assert calls["padra_DecodeAttentionSplits"](kv, 1, 4, 0, 0) == 32
 
 
+@pytest.mark.parametrize("wrong", [1.9, 2.0, "2", b"2", None, np.float32(2), [2]])
+def test_numbers_are_what_ctypes_takes(wrong):
+    """Counts are integers (anything with __index__), as through ctypes: nothing is truncated or
+    parsed.  eps takes a number, not its text."""
+    scratch, lib = abi.fast()["padra_DecodeAttentionScratch"], abi.lib()
+    for at in range(4):
+        args = [2, 2, 32, 32]
+        args[at] = wrong
+        with pytest.raises(ctypes.ArgumentError):
+            lib.padra_DecodeAttentionScratch(*args)
+        with pytest.raises(TypeError):
+            scratch(*args)
+    for right in (2, True, np.int64(2), (1 << 32) + 2, -1):
+        args = (2, right, 32, 32)
+        assert scratch(*args) == lib.padra_DecodeAttentionScratch(*args)
+    if not isinstance(wrong, (float, np.floating)):
+        x = _OnGpu()
+        with pytest.raises(TypeError):
+            abi.fast()["padra_ResidualPostNorm"](x, x, x, x, x, 1, 128, wrong, 128, None, x, 0)
+
+
 @pytest.mark.gpu
 def test_tensors_streams_and_status():
     class Sub(torch.Tensor):
