@@ -34,6 +34,8 @@ class _Calls:
     a nonzero status PadraError."""
 
     def __getattr__(self, name):
+        if not name.startswith("padra_") or name not in abi.fast():
+            raise AttributeError(name)
         self.__dict__.update(abi.fast())
         return self.__dict__[name]
 

@@ -87,6 +87,14 @@ def test_descriptors_are_their_own_structures():
     assert calls["padra_DecodeAttentionSplits"](kv, 1, 4, 0, 0) == 32
 
 
+def test_entry_points_by_name():
+    """Any other attribute is absent, and asking for it loads nothing."""
+    calls = ops._Calls()
+    assert not hasattr(calls, "__wrapped__") and not calls.__dict__
+    assert calls.padra_DecodeAttentionScratch(2, 2, 32, 32) > 0
+    assert not hasattr(calls, "padra_Nothing")
+
+
 @pytest.mark.parametrize("wrong", [1.9, 2.0, "2", b"2", None, np.float32(2), [2]])
 def test_numbers_are_what_ctypes_takes(wrong):
     """Counts are integers (anything with __index__), as through ctypes: nothing is truncated or
