@@ -277,8 +277,8 @@ __device__ __forceinline__ bool q8_scale_fast(float scale) {
 }
 
 // The values code * scale of a word of four codes (kv_q8::Decode), with the least code seen
-// (as a float; -128 is the code the reference rejects).  The caller gives keys past the
-// window zero codes and a unit scale, as the reference stages them.  Each code is one
+// (as a float; -128 is the code the reference rejects).  Keys past the window come with the last
+// key's row, whose codes are checked anyway.  Each code is one
 // v_cvt_f32_i32 with a sign-extended byte select; min(min(least, a), b) is one v_min3_f32.
 __device__ __forceinline__ void q8_values4(uint32_t w, float scale, float *f, float &least) {
 #pragma unroll
@@ -376,8 +376,8 @@ __global__ __launch_bounds__(64 * W) void k_attn_mx(AttnArgs a) {
   //  K: load m is key lane / KL + 64 / KL m, 16 bytes at chunk lane % KL of the row.
   //  V: BF16 m = 4 h + p is key 16 h + 4 grp + p, dimensions 8 col ..; q8 m is key
   //  4 (lane / 8) + m, dimensions 16 (lane % 8) ...
-  // Window offsets past the last key read the last key's row (the reference zero-fills
-  // them; their scores are masked to -inf, so their probabilities are 0).
+  // Window offsets past the last key read the last key's row (the reference zero-fills them);
+  // their scores are masked to -inf, so their probabilities are 0, and their V values zeroed.
   constexpr int KL = Q8 ? 8 : 16, CH = Q8 ? 4 : 8;
   uint4 kw[CH], vw[CH];
   float ksc[2], vsc[4]; // q8: scales of keys 16 h + col (K) and of this lane's V keys
@@ -398,13 +398,23 @@ __global__ __launch_bounds__(64 * W) void k_attn_mx(AttnArgs a) {
         ksc[h] = *reinterpret_cast<const float *>(sbytes + (size_t)row_of(tile, 16 * h + col) * scale_bytes);
     }
   };
+  auto v_key = [&](int m) { return 4 * (lane / KL) + (Q8 ? m : 16 * (m >> 2) + (m & 3)); };
   auto load_v = [&](int tile) {
 #pragma unroll
     for (int m = 0; m < CH; ++m) {
-      const uint32_t r = row_of(tile, 4 * (lane / KL) + (Q8 ? m : 16 * (m >> 2) + (m & 3)));
+      const uint32_t r = row_of(tile, v_key(m));
       vw[m] = ld_nt(reinterpret_cast<const uint4 *>(vbytes + part + (size_t)r * row_bytes));
       if constexpr (Q8)
         vsc[m] = *reinterpret_cast<const float *>(sbytes + 4 + (size_t)r * scale_bytes);
+    }
+  };
+  auto drop_v = [&](int left) { // zeroes the V rows of a tile's keys from `left`
+#pragma unroll
+    for (int m = 0; m < CH; ++m) {
+      const uint32_t keep = v_key(m) < left ? ~0u : 0u;
+      vw[m] = make_uint4(vw[m].x & keep, vw[m].y & keep, vw[m].z & keep, vw[m].w & keep);
+      if constexpr (Q8)
+        vsc[m] = keep ? vsc[m] : 1.f;
     }
   };
   if (begin + wave < end) { // wave-uniform
@@ -446,9 +456,12 @@ __global__ __launch_bounds__(64 * W) void k_attn_mx(AttnArgs a) {
     // loaded as soon as the registers are free (K once it is in LDS, V likewise).  The last
     // tile is code of its own: with the loads under a condition the compiler can only wait
     // for all of them at once, which exposed the latency of the tile just issued
-    // (W = 1: 148 -> 211 us at 131072 keys).
-    auto scores = [&](auto more) {
-      constexpr bool MORE = decltype(more)::value;
+    // (W = 1: 148 -> 211 us at 131072 keys).  So is a tile that the window's end cuts (CUT): its
+    // keys past the end have no V row, and an infinity of the last key's row, which they read,
+    // times their probability 0 would be NaN.  (Cleared in the last tile's code, with a test or
+    // for every one, 8 sequences to 8000 keys took 23.5 -> 23.7-23.9 us, so 23.6.)
+    auto scores = [&](auto more, auto cut) {
+      constexpr bool MORE = decltype(more)::value, CUT = decltype(cut)::value;
       const int left = n - tile * kKeys; // keys of this tile inside the window (may be >= 32)
       // Scores: lane holds row col, keys 16 h + 4 grp + i.
       f32x4_t s[2] = {f32x4_t{0.f, 0.f, 0.f, 0.f}, f32x4_t{0.f, 0.f, 0.f, 0.f}};
@@ -503,6 +516,8 @@ __global__ __launch_bounds__(64 * W) void k_attn_mx(AttnArgs a) {
                 fine = fine && q8_check16(kq[8 * (16 * h + col) + ((4 * u + grp) ^ (col >> 1))],
                                           kscale[h]);
         }
+        if constexpr (CUT)
+          drop_v(left);
         const int t7 = lane & 7, j = lane >> 3;
         uint2 *dst = &vq[wave][j][(16 * t7) ^ ((j & 1) << 4)];
 #pragma unroll
@@ -542,6 +557,8 @@ __global__ __launch_bounds__(64 * W) void k_attn_mx(AttnArgs a) {
 #pragma unroll
           for (int t = 0; t < 4; ++t)
             s[h] = mfma_bf16(kq[16 * (16 * h + col) + ((4 * t + grp) ^ col)], qb[t], s[h]);
+        if constexpr (CUT)
+          drop_v(left);
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
           const uint4 *p = &vw[4 * h];
@@ -576,10 +593,12 @@ __global__ __launch_bounds__(64 * W) void k_attn_mx(AttnArgs a) {
       tmax = fmaxf(tmax, lane_xor<16>(tmax));
       tmax = fmaxf(tmax, lane_xor<32>(tmax));
     };
-    if (tile + W < end) // wave-uniform
-      scores(std::true_type{});
+    if (tile + W < end) // wave-uniform, all three
+      scores(std::true_type{}, std::false_type{});
+    else if (tile * kKeys + kKeys > n && tile < end)
+      scores(std::false_type{}, std::true_type{});
     else if (tile < end)
-      scores(std::false_type{});
+      scores(std::false_type{}, std::false_type{});
     if (W > 1 && grp == 0)
       tile_max[wave][col] = tmax; // -inf without a tile
     // The running maximum at this wave's tile (every tile of the round before it counted),

@@ -169,3 +169,55 @@ def test_decode_attention_units(fmt, seqs):
     assert run(slice(0, seqs), states, out) == 1
     for i in range(seqs):
         assert torch.equal(out[i], torch.full_like(out[i], 77) if i in refused else alone[i]), i
+
+
+@pytest.mark.parametrize("fmt", [abi.KV_BF16, abi.KV_Q8])
+@pytest.mark.parametrize("local", [False, True])
+def test_decode_attention_infinity_in_the_last_row(oracle, fmt, local):
+    """An infinity in the V row of the window's last key comes out as that infinity in its
+    dimension (and raises the flag), also where the last tile has keys past the window: those have
+    no V row at all.  Batches of 3 and 40 (several waves a split, one)."""
+    hq, hkv, capacity = 32, 4, 1024
+    windows = [1, 31, 32, 33, 100, 1000, 1023, 1024]
+    print(f"[case] attention infinity fmt={fmt} local={local}", flush=True)
+    rng = np.random.default_rng(5)
+    n = len(windows)
+    q = synth.bf16_bits(rng.standard_normal((n, hq, 128)).astype(np.float32))
+    kc, vc = _rows(fmt, rng, n * capacity), _rows(fmt, rng, n * capacity)
+    sc = rng.uniform(.005, .02, (n * capacity, hkv, 2)).astype(np.float32)
+    for i, w in enumerate(windows):
+        last = i * capacity + w - 1
+        if fmt == abi.KV_BF16:
+            vc[last, 7::128] = np.uint16(0xff80).view(np.int16)
+        else:
+            vc[last] = 0
+            vc[last, 7::128] = -100
+            sc[last, :, 1] = 1e37
+    dense = kc.view(np.uint16), vc.view(np.uint16)
+    if fmt == abi.KV_Q8:
+        with np.errstate(over="ignore"):
+            dense = [synth.bf16_bits(c.reshape(-1, hkv, 128).astype(np.float32) * sc[..., i:i + 1])
+                     .reshape(-1, 512) for i, c in enumerate((kc, vc))]
+    for size in (3, 40):
+        pick = np.arange(size) % n
+        rows = np.concatenate([np.arange(i * capacity, (i + 1) * capacity) for i in pick])
+        kd, vd, sd, qd = (torch.from_numpy(np.ascontiguousarray(a)).cuda()
+                          for a in (kc[rows], vc[rows], sc[rows], q[pick].view(np.int16)))
+        states = torch.tensor([[5, windows[i] - 1, capacity, 10, windows[i] - 1,
+                                min(windows[i] - 1, 1024), 0, 0] for i in pick], dtype=torch.int32)
+        bad = torch.zeros(1, dtype=torch.int32, device="cuda")
+        out = torch.empty_like(qd)
+        ops.DecodeAttention(qd, ops.kv_cache(fmt, kd, vd, capacity, scales=sd, seq_stride=capacity),
+                            out, ops.positions_decode(states.cuda(), maximum=capacity), bad,
+                            kv_heads=hkv, local=local)
+        torch.cuda.synchronize()
+        assert bad.item() == 1
+        got = synth.bf16_to_f32(out.cpu().numpy().view(np.uint16))
+        for s, i in enumerate(pick):
+            k, v = (p[i * capacity:(i + 1) * capacity] for p in dense)
+            want, _, wbad = oracle.decode_attention(q[i], k, v, windows[i] - 1, local=local)
+            want = synth.bf16_to_f32(want)
+            assert wbad and np.isneginf(want[:, 7]).all()
+            assert np.isneginf(got[s][:, 7]).all(), (size, windows[i])
+            rest = np.arange(128) != 7
+            assert np.isfinite(want[:, rest]).all() and np.isfinite(got[s][:, rest]).all()
