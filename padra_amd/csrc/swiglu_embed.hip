@@ -101,8 +101,9 @@ __device__ __forceinline__ void swiglu8(const uint32_t (&gp)[4], const float (&u
   float most = 0.f;
 #pragma unroll
   for (int k = 0; k < 8; ++k) {
-    r[k] = __uint_as_float(s[k] << 16) * u[k]; // finite operands: no NaN for fmaxf to drop
-    most = fmaxf(most, fabsf(r[k]));
+    r[k] = __uint_as_float(s[k] << 16) * u[k];
+    // keeps a NaN, which a table that holds one gives (v_maximum3_f32)
+    most = __builtin_elementwise_maximum(most, fabsf(r[k]));
   }
   fine = fine && bf16_finite(most);
 #pragma unroll

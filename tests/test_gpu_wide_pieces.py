@@ -76,6 +76,26 @@ def test_swiglu_f32_inexact_gate():
     assert torch.equal(out, want)
 
 
+@pytest.mark.parametrize("act", ["bf16", "f32"])
+def test_swiglu_nan_in_the_table(act):
+    """A product that is NaN raises the flag also where operands and gate are ordinary: with a
+    table that holds a NaN (one never built, or overwritten)."""
+    table = torch.empty(65536, dtype=torch.int16, device="cuda")
+    ops.SiluTableBuild(table)
+    table[0x3F80] = 0x7FC0  # silu(1)
+    dtype = torch.bfloat16 if act == "bf16" else torch.float32
+    g = torch.full((1024,), 2., device="cuda", dtype=dtype)
+    up, out = torch.ones_like(g), torch.empty_like(g)
+    for at, flag in ((None, 0), (0, 1), (511, 1), (700, 1)):
+        g.fill_(2.)
+        if at is not None:
+            g[at] = 1.
+        bad = torch.zeros(1, dtype=torch.int32, device="cuda")
+        ops.SwiGLU(g, up, out, table, bad)
+        assert bad.item() == flag, at
+        assert out.isnan().sum().item() == flag
+
+
 @pytest.mark.parametrize("hidden", [1024, 1152, 2048, 2304, 4096, 4608])
 @pytest.mark.parametrize("rows,fp8", [(37, False), (37, True), (2048, True)])
 def test_combine_norm_f32_equals_bf16(hidden, rows, fp8):
