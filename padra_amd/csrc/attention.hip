@@ -377,7 +377,7 @@ __global__ __launch_bounds__(64 * W) void k_attn_mx(AttnArgs a) {
   //  V: BF16 m = 4 h + p is key 16 h + 4 grp + p, dimensions 8 col ..; q8 m is key
   //  4 (lane / 8) + m, dimensions 16 (lane % 8) ...
   // Window offsets past the last key read the last key's row (the reference zero-fills them);
-  // their scores are masked to -inf, so their probabilities are 0, and their V values zeroed.
+  // their scores are masked to -inf, so their probabilities are 0, and their V values finite.
   constexpr int KL = Q8 ? 8 : 16, CH = Q8 ? 4 : 8;
   uint4 kw[CH], vw[CH];
   float ksc[2], vsc[4]; // q8: scales of keys 16 h + col (K) and of this lane's V keys
@@ -406,15 +406,6 @@ __global__ __launch_bounds__(64 * W) void k_attn_mx(AttnArgs a) {
       vw[m] = ld_nt(reinterpret_cast<const uint4 *>(vbytes + part + (size_t)r * row_bytes));
       if constexpr (Q8)
         vsc[m] = *reinterpret_cast<const float *>(sbytes + 4 + (size_t)r * scale_bytes);
-    }
-  };
-  auto drop_v = [&](int left) { // zeroes the V rows of a tile's keys from `left`
-#pragma unroll
-    for (int m = 0; m < CH; ++m) {
-      const uint32_t keep = v_key(m) < left ? ~0u : 0u;
-      vw[m] = make_uint4(vw[m].x & keep, vw[m].y & keep, vw[m].z & keep, vw[m].w & keep);
-      if constexpr (Q8)
-        vsc[m] = keep ? vsc[m] : 1.f;
     }
   };
   if (begin + wave < end) { // wave-uniform
@@ -456,10 +447,12 @@ __global__ __launch_bounds__(64 * W) void k_attn_mx(AttnArgs a) {
     // loaded as soon as the registers are free (K once it is in LDS, V likewise).  The last
     // tile is code of its own: with the loads under a condition the compiler can only wait
     // for all of them at once, which exposed the latency of the tile just issued
-    // (W = 1: 148 -> 211 us at 131072 keys).  So is a tile that the window's end cuts (CUT): its
-    // keys past the end have no V row, and an infinity of the last key's row, which they read,
-    // times their probability 0 would be NaN.  (Cleared in the last tile's code, with a test or
-    // for every one, 8 sequences to 8000 keys took 23.5 -> 23.7-23.9 us, so 23.6.)
+    // (W = 1: 148 -> 211 us at 131072 keys).  So is, in BF16, a tile that the window's end cuts
+    // (CUT): its keys past the end have no V row, and an infinity of the last key's row, which they
+    // read, times their probability 0 would be NaN.  (Cleared in the last tile's code, with a test
+    // or for every one, 8 sequences to 8000 keys took 23.5 -> 23.7-23.9 us, so 23.6.)  In q8 a scale
+    // of 1 for those keys does it, in the last tile's code: with code of its own 12 sequences to
+    // 65536 keys took 154 us, 16 to 8000 35.0, so 152 and 34.7.
     auto scores = [&](auto more, auto cut) {
       constexpr bool MORE = decltype(more)::value, CUT = decltype(cut)::value;
       const int left = n - tile * kKeys; // keys of this tile inside the window (may be >= 32)
@@ -516,8 +509,11 @@ __global__ __launch_bounds__(64 * W) void k_attn_mx(AttnArgs a) {
                 fine = fine && q8_check16(kq[8 * (16 * h + col) + ((4 * u + grp) ^ (col >> 1))],
                                           kscale[h]);
         }
-        if constexpr (CUT)
-          drop_v(left);
+        if constexpr (!MORE) { // keys past the window: a finite value for any scale
+#pragma unroll
+          for (int m = 0; m < 4; ++m)
+            vsc[m] = v_key(m) < left ? vsc[m] : 1.f;
+        }
         const int t7 = lane & 7, j = lane >> 3;
         uint2 *dst = &vq[wave][j][(16 * t7) ^ ((j & 1) << 4)];
 #pragma unroll
@@ -557,8 +553,13 @@ __global__ __launch_bounds__(64 * W) void k_attn_mx(AttnArgs a) {
 #pragma unroll
           for (int t = 0; t < 4; ++t)
             s[h] = mfma_bf16(kq[16 * (16 * h + col) + ((4 * t + grp) ^ col)], qb[t], s[h]);
-        if constexpr (CUT)
-          drop_v(left);
+        if constexpr (CUT) {
+#pragma unroll
+          for (int m = 0; m < CH; ++m) {
+            const uint32_t keep = v_key(m) < left ? ~0u : 0u;
+            vw[m] = make_uint4(vw[m].x & keep, vw[m].y & keep, vw[m].z & keep, vw[m].w & keep);
+          }
+        }
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
           const uint4 *p = &vw[4 * h];
@@ -595,7 +596,7 @@ __global__ __launch_bounds__(64 * W) void k_attn_mx(AttnArgs a) {
     };
     if (tile + W < end) // wave-uniform, all three
       scores(std::true_type{}, std::false_type{});
-    else if (tile * kKeys + kKeys > n && tile < end)
+    else if (!Q8 && tile * kKeys + kKeys > n && tile < end)
       scores(std::false_type{}, std::true_type{});
     else if (tile < end)
       scores(std::false_type{}, std::false_type{});
