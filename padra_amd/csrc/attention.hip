@@ -301,7 +301,7 @@ __device__ __forceinline__ void q8_values8(uint32_t w0, uint32_t w1, float scale
 }
 
 // kv_q8::Decode's checks on a chunk whose scale failed q8_scale_fast: a valid scale and
-// every code * scale finite in BF16.
+// every code * scale finite in BF16, which the largest |code| decides.
 __device__ __forceinline__ bool q8_check16(uint4 c, float scale) {
   uint32_t w[4] = {c.x, c.y, c.z, c.w};
   // An opaque copy: the compiler would otherwise keep every decoded value of the tile in
@@ -309,15 +309,13 @@ __device__ __forceinline__ bool q8_check16(uint4 c, float scale) {
 #pragma unroll
   for (int i = 0; i < 4; ++i)
     asm volatile("" : "+v"(w[i]));
-  bool ok = isfinite(scale) && scale > 0.f;
+  float most = 0.f;
 #pragma unroll
   for (int i = 0; i < 4; ++i)
 #pragma unroll
-    for (int b = 0; b < 4; ++b) {
-      const float v = (float)(int8_t)((w[i] >> (8 * b)) & 0xffu) * scale;
-      ok = ok & ((pack2(v, 0.f) & 0x7f80u) != 0x7f80u);
-    }
-  return ok;
+    for (int b = 0; b < 4; ++b)
+      most = fmaxf(most, fabsf((float)(int8_t)((w[i] >> (8 * b)) & 0xffu)));
+  return isfinite(scale) && scale > 0.f && most * scale < 0x1.ffp127f;
 }
 
 // Slot of dimension d in a staged V row.  Each staging lane writes its dimension pairs at
@@ -334,8 +332,14 @@ template <bool Q8> __device__ __forceinline__ int vq_slot(int d) {
   }
 }
 
-template <class T, bool Q8, int W>
-__global__ __launch_bounds__(64 * W) void k_attn_mx(AttnArgs a) {
+// DENSE: for q8 launches of more one-wave workgroups than two on each SIMD (2048), held to the
+// registers of three (168 VGPRs, no spill, for 190): the decode is arithmetic, which a third wave
+// fills.  64 sequences (us): to 131072 keys (16 heads) 788 -> 727, to 32768 238 -> 222, to 8000 keys (32
+// heads) 96.9 -> 90.0; 24 to 8000 keys 50.6 -> 48.5.  In smaller launches two a SIMD is all there is
+// and the order that this takes costs 3-5%: 12 sequences to 65536 keys 154 -> 162.
+template <class T, bool Q8, int W, bool DENSE = false>
+__global__ __launch_bounds__(64 * W, DENSE ? 3 : 1) void k_attn_mx(AttnArgs a) {
+  constexpr bool HELD = Q8 && (W > 1 || DENSE);
   constexpr int NB = 8 / W; // 16-dimension blocks of the output per wave
   const int G = a.group;
   // Per tile of the round: (V[4j][d], V[4j+1][d]), (V[4j+2][d], V[4j+3][d]) at slot
@@ -473,8 +477,8 @@ __global__ __launch_bounds__(64 * W) void k_attn_mx(AttnArgs a) {
           load_k(tile + W);
           issue_point();
         }
-        // Decoded a chunk at a time: the scheduling barriers keep one chunk's values in
-        // registers, not all of them (256 VGPRs and spills without).
+        // Decoded a chunk at a time where HELD: the scheduling barriers keep one chunk's values in
+        // registers, not all of them.
         float least = 0.f;
         // Whether some key's scale needs every value checked (rare: huge or invalid scales).
         const bool kslow = __ballot(!q8_scale_fast(kscale[0]) || !q8_scale_fast(kscale[1])) != 0;
@@ -497,7 +501,7 @@ __global__ __launch_bounds__(64 * W) void k_attn_mx(AttnArgs a) {
               w[4 + e] = pack2(f[2 * e], f[2 * e + 1]);
             s[h] = mfma_bf16(make_uint4(w[0], w[1], w[2], w[3]), qb[2 * u], s[h]);
             s[h] = mfma_bf16(make_uint4(w[4], w[5], w[6], w[7]), qb[2 * u + 1], s[h]);
-            if constexpr (W > 1)
+            if constexpr (HELD)
               __builtin_amdgcn_sched_barrier(0);
           }
         if (kslow) { // one rare branch, not one per chunk, which would cut the code above apart
@@ -528,7 +532,7 @@ __global__ __launch_bounds__(64 * W) void k_attn_mx(AttnArgs a) {
             *reinterpret_cast<uint4 *>(dst + 2 * ((2 * i + e / 2 + t7) & 7)) =
                 make_uint4(pack2(f[0][e], f[1][e]), pack2(f[2][e], f[3][e]),
                            pack2(f[0][e + 1], f[1][e + 1]), pack2(f[2][e + 1], f[3][e + 1]));
-          if constexpr (W > 1)
+          if constexpr (HELD)
             __builtin_amdgcn_sched_barrier(0);
         }
         fine = fine && least > -128.f;
@@ -649,6 +653,9 @@ __global__ __launch_bounds__(64 * W) void k_attn_mx(AttnArgs a) {
         const int d = vq_slot<Q8>(16 * (NB * wave + b) + col) ^ ((grp & 1) << 4);
         const uint2 v0 = vq[t][grp][d], v1 = vq[t][4 + grp][d];
         o[b] = mfma_bf16(pt, make_uint4(v0.x, v0.y, v1.x, v1.y), o[b] * rescale);
+        if constexpr (HELD)
+          if ((b & 3) == 3)
+            __builtin_amdgcn_sched_barrier(0);
       }
     };
     if (count == W) { // block-uniform; without a test per tile its LDS reads overlap
@@ -1793,6 +1800,8 @@ int decode_attention(void *stream, const void *q, const padra_KVCache *kv, void 
       else if (wgs <= 1024 && !local) // a local ring's split has two tiles or so: 15.2 us
                                       // with two waves, 14.9 with one (12 sequences)
         split(q8tag, std::integral_constant<int, 2>{});
+      else if (decltype(q8tag)::value && wgs > 2048) // (k_attn_mx, DENSE)
+        hipLaunchKernelGGL((k_attn_mx<T, true, 1, true>), split_grid, dim3(64), 0, s, a);
       else
         split(q8tag, std::integral_constant<int, 1>{});
     };

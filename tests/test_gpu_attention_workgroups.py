@@ -221,3 +221,66 @@ def test_decode_attention_infinity_in_the_last_row(oracle, fmt, local):
             assert np.isneginf(got[s][:, 7]).all(), (size, windows[i])
             rest = np.arange(128) != 7
             assert np.isfinite(want[:, rest]).all() and np.isfinite(got[s][:, rest]).all()
+
+
+def _edge_scales(code):
+    """The largest scale at which code * scale stays finite in BF16, and the next one (fp32)."""
+    limit, s = np.float32(float.fromhex("0x1.ffp127")), np.float32(float.fromhex("0x1.ffp127") / code)
+    s = np.nextafter(s, np.float32(0))
+    while np.float32(code) * s < limit:
+        s = np.nextafter(s, np.float32(np.inf))
+    while not np.float32(code) * s < limit:
+        s = np.nextafter(s, np.float32(0))
+    return s, np.nextafter(s, np.float32(np.inf))
+
+
+@pytest.mark.parametrize("act", ["bf16", "f32"])
+@pytest.mark.parametrize("window", [1, 40, 1024])
+def test_decode_attention_q8_values(act, window):
+    """kv_q8::Decode's checks of a cache row's scale and codes, K and V, in launches of 1, 16 and 20
+    sequences (8 waves a split, one, one held to fewer registers): the largest scale that leaves
+    code * scale finite in BF16 passes, the next one, an invalid scale and code -128 raise the flag.
+    What passes has the same bits in every batch."""
+    print(f"[case] attention q8 values act={act} window={window}", flush=True)
+    hq, hkv, cap, seqs = 8, 4, 1024, 20
+    g = torch.Generator(device="cuda").manual_seed(window)
+    # small queries: a score of the largest values stays finite
+    q = (torch.randn((seqs, hq, 128), generator=g, device="cuda") * 2.**-110).bfloat16()
+    q = q.float() if act == "f32" else q
+    planes = [torch.randint(-127, 128, (seqs * cap, 512), generator=g, device="cuda",
+                            dtype=torch.int8) for _ in range(2)]
+    sc = torch.rand((seqs * cap, hkv, 2), generator=g, device="cuda") * .01 + .01
+    states = torch.tensor([[5, window - 1, cap, 10, window - 1, window - 1, 0, 0]] * seqs,
+                          dtype=torch.int32, device="cuda")
+    cases = [(0, float(s), True) for s in (np.nan, np.inf, 0., -1.)] + [(-128, .01, True)]
+    for code in (127, 100, 1):
+        fits, over = _edge_scales(code)
+        cases += [(code, float(fits), False), (-code, float(over), True)]
+
+    def run(n):
+        bad = torch.zeros(1, dtype=torch.int32, device="cuda")
+        out = torch.empty_like(q[:n])
+        at = slice((seqs - n) * cap, None)  # the last n sequences
+        kv = ops.kv_cache(abi.KV_Q8, planes[0][at], planes[1][at], cap, scales=sc[at],
+                          seq_stride=cap)
+        ops.DecodeAttention(q[seqs - n:], kv, out, ops.positions_decode(states[:n], maximum=cap),
+                            bad, kv_heads=hkv)
+        return bad.item(), out
+
+    for plane in (0, 1):
+        for code, scale, flagged in cases:
+            row = seqs * cap - cap + window - 1  # the last key of the last sequence
+            before = planes[plane][row].clone(), sc[row].clone()
+            planes[plane][row] = 0
+            planes[plane][row, 5::128] = code
+            sc[row, :, plane] = scale
+            results = [run(n) for n in (1, 16, 20)]
+            planes[plane][row], sc[row] = before
+            assert [b for b, _ in results] == [int(flagged)] * 3, (plane, code, scale)
+            if not flagged:
+                assert torch.equal(results[0][1][-1], results[1][1][-1])
+                assert torch.equal(results[0][1][-1], results[2][1][-1])
+                assert torch.equal(results[1][1], results[2][1][-16:])
+                assert results[0][1].isfinite().all()
+    bad, out = run(20)
+    assert bad == 0 and out.isfinite().all()
