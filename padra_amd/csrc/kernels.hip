@@ -615,8 +615,8 @@ int chain(hipStream_t s, const uint16_t *gather, int vocab, const int32_t *ids, 
 } // namespace
 
 namespace {
-// The chain on fp32 activations (the reference's buffers), in one launch but for one corner
-// (below): up to head_wave_tokens of norm-row waves and per-head Q/K waves.
+// The chain on fp32 activations (the reference's buffers), in one launch: up to head_wave_tokens of
+// norm-row waves and per-head Q/K waves, above of norm-row waves and four-lanes-per-head ones.
 int chain_f32(hipStream_t s, void *x, const void *residual, void *normalized,
               const uint16_t *gamma, int hidden, int tree, float *statistics, void *q, void *k,
               const void *v, const uint16_t *qn, const uint16_t *kn, const uint16_t *table,
@@ -651,29 +651,23 @@ int chain_f32(hipStream_t s, void *x, const void *residual, void *normalized,
                            dim3((unsigned)waves), dim3(64), 0, s, n, a, norm_waves, waves);
         return launched();
       }
-      // Above, one launch too, norm rows and then four-lanes-per-head Q/K waves.  The norm rows
-      // get the Q/K waves' registers there (142 VGPRs, 3 waves per SIMD, against 89 and 5
-      // alone), but the Q/K waves, whose chain alone lasts 6-7 us, start while the norm rows still
+      // The norm rows get the Q/K waves' registers here (142 VGPRs, 3 waves per SIMD, against 89 and
+      // 5 alone), but the Q/K waves, whose chain alone lasts 6-7 us, start while the norm rows still
       // stream.  One kernel against two on the stream (us; BF16 / q8 / rotated q8_0 cache):
       //   hidden 2048, 16 heads, 512 tokens  8.7 : 11.9  11.8 : 14.7  11.3 : 14.5
       //                         1000        13.7 : 14.9  15.6 : 17.2  15.2 : 16.9
-      //                         2048        22.8 : 22.7  24.1 : 25.4  25.0 : 26.5
+      //                         2048        21.0 : 21.3  24.1 : 25.4  25.0 : 26.5
       //   hidden 2304, 32 heads, 512 tokens 10.1 : 13.2  12.5 : 15.5  12.1 : 15.3
       //                         2048        30.2 : 33.4  31.4 : 34.7  31.7 : 35.0
-      // Only where few heads and no encoding leave the Q/K part short beside many norm rows do
-      // two kernels come out ahead (16 heads, BF16 cache: 1400 tokens 17.5 : 17.7, 2048 tokens 22.8 :
-      // 22.7 here and 22.2 : 21.3 with all inputs cold): from 1792 tokens of at most 20 heads.
-      if (fmt.value <= PADRA_KV_BF16 && tokens >= 1792 && q_heads + kv_heads <= 20) {
-        hipLaunchKernelGGL((k_norm<vt.value, j.value, float, true>), dim3((unsigned)norm_waves),
-                           dim3(64), 0, s, n);
-        const int st2 = launched();
-        if (st2)
-          return st2;
-        hipLaunchKernelGGL((k_qk<float, fmt.value>),
-                           dim3((unsigned)qk_wave_count<fmt.value>(tokens, q_heads, kv_heads)),
-                           dim3(64), 0, s, a);
-        return launched();
-      }
+      //   BF16 cache, warm and cold (all inputs from HBM):
+      //   hidden 2048, 16 heads, 1792 tokens 18.6 : 19.5  20.4 : 20.7
+      //                         2048         21.0 : 21.3  22.6 : 22.5
+      //                         4096         39.3 : 42.8  42.3 : 45.7
+      //   hidden 2304, 16 heads, 2048 tokens 22.3 : 21.5  24.2 : 24.1
+      //                24 heads, 1400 tokens 17.9 : 18.4  20.0 : 19.4
+      //                32 heads, 1024 tokens 14.4 : 16.6  18.0 : 17.5
+      // Two kernels are level or up to 4% ahead only where the Q/K waves just fill the chip once
+      // (3072 of them) and the norm rows beside them start a second round: too narrow for a rule.
       const long long waves = norm_waves + qk_wave_count<fmt.value>(tokens, q_heads, kv_heads);
       hipLaunchKernelGGL((k_chain<vt.value, j.value, fmt.value, false, float>),
                          dim3((unsigned)waves), dim3(64), 0, s, n, a, norm_waves, waves);
