@@ -659,15 +659,13 @@ int chain_f32(hipStream_t s, void *x, const void *residual, void *normalized,
       //                         2048        21.0 : 21.3  24.1 : 25.4  25.0 : 26.5
       //   hidden 2304, 32 heads, 512 tokens 10.1 : 13.2  12.5 : 15.5  12.1 : 15.3
       //                         2048        30.2 : 33.4  31.4 : 34.7  31.7 : 35.0
-      //   BF16 cache, warm and cold (all inputs from HBM):
-      //   hidden 2048, 16 heads, 1792 tokens 18.6 : 19.5  20.4 : 20.7
-      //                         2048         21.0 : 21.3  22.6 : 22.5
-      //                         4096         39.3 : 42.8  42.3 : 45.7
-      //   hidden 2304, 16 heads, 2048 tokens 22.3 : 21.5  24.2 : 24.1
-      //                24 heads, 1400 tokens 17.9 : 18.4  20.0 : 19.4
-      //                32 heads, 1024 tokens 14.4 : 16.6  18.0 : 17.5
-      // Two kernels are level or up to 4% ahead only where the Q/K waves just fill the chip once
-      // (3072 of them) and the norm rows beside them start a second round: too narrow for a rule.
+      //   BF16 cache, all inputs from HBM, 128-thread tree:
+      //   hidden 2048,  8 heads, 3072 tokens 28.3 : 29.6    16 heads, 1700 tokens 19.7 : 19.6
+      //                16 heads, 2048        22.8 : 23.4    16 heads, 3072        32.3 : 35.0
+      //                24 heads, 1400        18.9 : 18.9    24 heads, 1550        20.2 : 21.8
+      //   hidden 2304, 16 heads, 2048        23.5 : 24.9    32 heads, 900         16.3 : 16.3
+      // Where the Q/K waves just fill the chip once (3072 of them: 16 heads x 2048 tokens, 24 x
+      // 1536) two kernels come closest, and with other buffers they have been up to 4% ahead.
       const long long waves = norm_waves + qk_wave_count<fmt.value>(tokens, q_heads, kv_heads);
       hipLaunchKernelGGL((k_chain<vt.value, j.value, fmt.value, false, float>),
                          dim3((unsigned)waves), dim3(64), 0, s, n, a, norm_waves, waves);
