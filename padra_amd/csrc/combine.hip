@@ -10,6 +10,7 @@
 #include <stdio.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "norm_fp8.h"
 
@@ -33,6 +34,7 @@ template <class T, int PIECE> __device__ __forceinline__ void load8_piece(const 
   if constexpr (PIECE == 4) {
     ActIO<T>::load8(p, v);
   } else {
+    static_assert(std::is_same<T, float>::value, "a piece is four fp32 columns");
     const uint4 a = ld_nt(reinterpret_cast<const uint4 *>(p));
     const uint4 b = ld_nt(reinterpret_cast<const uint4 *>(p + PIECE));
     const uint32_t w[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
@@ -113,13 +115,14 @@ __global__ __launch_bounds__(256) void k_combine(T *x, const T *down, const floa
 // BF16 rows take k_combine_norm_wide, whose order-free sum makes every wave's finish cheap.
 constexpr int kCombineWaves = 4;
 
-// Combine + RMSNorm (+ FP8): W waves per row.  The combine runs in the natural layout
-// (lane l takes columns 8l..8l+7 of each 512-column chunk, 16-byte accesses; wave w takes
-// chunks w, w + W, ...), its BF16 results go through LDS, and wave 0 reads them back in
-// the 128-thread ownership layout (lane l: columns 2l, 2l+1 of each 128) for the norm.
-template <int J, class T, bool FP8, int W>
-__global__ __launch_bounds__(64 * W) void k_combine_norm(T *x, const T *down, const float *weights,
-                                                         NormFP8Args<T> a) {
+// Combine + RMSNorm (+ FP8) of fp32 rows: W waves per row.  Wave w takes the row's 512-column
+// chunks w, w + W, ..., lane l columns 4l .. 4l + 3 of each half of a chunk (16-byte accesses), the
+// BF16 results go through LDS, and wave 0 reads them back in the 128-thread ownership layout
+// (lane l: columns 2l, 2l+1 of each 128) for the norm.
+template <int J, bool FP8, int W>
+__global__ __launch_bounds__(64 * W) void k_combine_norm(float *x, const float *down,
+                                                         const float *weights,
+                                                         NormFP8Args<float> a) {
   constexpr int H = 128 * J, CHUNKS = (H + 511) / 512;
   __shared__ uint32_t v_lds[H / 2];
   const int row = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -131,15 +134,14 @@ __global__ __launch_bounds__(64 * W) void k_combine_norm(T *x, const T *down, co
   bool fine = true;
 #pragma unroll
   for (int i = 0; i < (CHUNKS + W - 1) / W; ++i) {
-    // a chunk's lane: columns 4l .. 4l + 3 and the same of its second half; a last chunk of 256
-    // columns has 8l .. 8l + 7 of its lower lanes
+    // a last chunk of 128 or 256 columns: 8l .. 8l + 7 of its lower lanes
     const int ch = wave + W * i;
     auto piece = [&](auto apart, int col) {
       constexpr int P = decltype(apart)::value;
-      T *xr = x + (size_t)row * H + col;
+      float *xr = x + (size_t)row * H + col;
       uint32_t out[4];
       bool f;
-      combine8<T, true, P>(xr, down + (size_t)row * kExperts * H + col, (size_t)H,
+      combine8<float, true, P>(xr, down + (size_t)row * kExperts * H + col, (size_t)H,
                            weights + (size_t)row * kExperts, out, f);
       st_wt(reinterpret_cast<uint4 *>(xr), make_uint4(out[0] << 16, out[0] & 0xffff0000u,
                                                       out[1] << 16, out[1] & 0xffff0000u));
@@ -166,7 +168,7 @@ __global__ __launch_bounds__(64 * W) void k_combine_norm(T *x, const T *down, co
 #pragma unroll
   for (int j = 0; j < J; ++j)
     vp[j] = v_lds[64 * j + lane];
-  norm_fp8_finish<J, T, FP8, true>(a, row, vp, gr);
+  norm_fp8_finish<J, float, FP8, true>(a, row, vp, gr);
 }
 
 // BF16 rows: the same combine, with the norm and the encoding spread over the W waves too.
@@ -482,11 +484,11 @@ extern "C" int padra_CombineNorm(void *stream, void *x, const void *down, const 
                              static_cast<const uint16_t *>(down), weights, a);
       } else {
         if (packed)
-          hipLaunchKernelGGL((k_combine_norm<j.value, T, true, kCombineWaves>), dim3(rows),
+          hipLaunchKernelGGL((k_combine_norm<j.value, true, kCombineWaves>), dim3(rows),
                              dim3(64 * kCombineWaves), 0, s,
                              static_cast<T *>(x), static_cast<const T *>(down), weights, a);
         else
-          hipLaunchKernelGGL((k_combine_norm<j.value, T, false, kCombineWaves>), dim3(rows),
+          hipLaunchKernelGGL((k_combine_norm<j.value, false, kCombineWaves>), dim3(rows),
                              dim3(64 * kCombineWaves), 0, s,
                              static_cast<T *>(x), static_cast<const T *>(down), weights, a);
       }

@@ -127,3 +127,24 @@ def test_combine_norm_f32_equals_bf16(hidden, rows, fp8):
             assert torch.allclose(one[9].float(), two[9].float(), equal_nan=True)
         else:
             assert torch.equal(one, two)
+
+
+@pytest.mark.parametrize("hidden", [1024, 1152, 2048, 2304, 4096, 4608])
+@pytest.mark.parametrize("act", [torch.bfloat16, torch.float32])
+def test_combine_norm_finite_rows_raise_no_flag(hidden, act):
+    """Every column of a row finite, up to the largest whose sums stay so: the flag stays down.  One
+    value that is not, in any lane of any chunk, raises it."""
+    rows = 3
+    g = torch.Generator(device="cuda").manual_seed(hidden)
+    weights = torch.full((rows, 8), .125, device="cuda")
+    gamma = torch.ones(hidden, device="cuda", dtype=torch.bfloat16)
+    x = torch.randn((rows, hidden), generator=g, device="cuda").to(torch.bfloat16).to(act)
+    down = torch.randn((rows, 8, hidden), generator=g, device="cuda").to(torch.bfloat16).to(act)
+    x[1] = 2.**55  # (the sum of its squares stays finite)
+    for at in [None, *range(0, hidden, 4)]:
+        a, d = x.clone(), down.clone()
+        if at is not None:
+            d[2, at % 8, at + at // 4 % 4] = float("inf") if at % 8 else float("nan")
+        y, bad = torch.empty_like(a), torch.zeros(1, dtype=torch.int32, device="cuda")
+        ops.CombineNorm(a, d, weights, y, gamma, bad)
+        assert bad.item() == (at is not None), at
