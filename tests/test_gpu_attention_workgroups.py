@@ -284,3 +284,98 @@ def test_decode_attention_q8_values(act, window):
                 assert results[0][1].isfinite().all()
     bad, out = run(20)
     assert bad == 0 and out.isfinite().all()
+
+
+def _q8_0_batch(rng, seqs, hq, cap, positions):
+    q = synth.bf16_bits((rng.standard_normal((seqs, hq, 128)) * 2).astype(np.float32))
+    kc, vc = _rows(abi.KV_Q8_0, rng, seqs * cap), _rows(abi.KV_Q8_0, rng, seqs * cap)
+    states = torch.tensor([[5, p, cap, 10, p, min(p, 1024), 0, 0] for p in positions],
+                          dtype=torch.int32)
+    kd, vd = torch.from_numpy(kc).cuda(), torch.from_numpy(vc).cuda()
+    qd = torch.from_numpy(q.view(np.int16)).cuda()
+
+    def run(some, splits, st=states):
+        rows = slice(some.start * cap, some.stop * cap)
+        out = torch.full((some.stop - some.start, hq, 128), 77, dtype=torch.int16, device="cuda")
+        bad = torch.zeros(1, dtype=torch.int32, device="cuda")
+        ops.DecodeAttention(qd[some], ops.kv_cache(abi.KV_Q8_0, kd[rows], vd[rows], cap, seq_stride=cap),
+                            out, ops.positions_decode(st[some].cuda(), maximum=cap), bad,
+                            splits=splits)
+        return out, bad.item()
+
+    return q, kc, vc, states, run
+
+
+@pytest.mark.parametrize("hq", [4, 8, 16, 32])
+def test_decode_attention_q8_0_whole_rows(oracle, hq):
+    """The q8_0 split of larger batches (a workgroup per split, its waves the KV heads) for every
+    number of query heads on a KV head: 9 sequences of 32 splits against the oracle and, bit for
+    bit, against each sequence alone (a workgroup per split and KV head)."""
+    print(f"[case] attention q8_0 whole rows hq={hq}", flush=True)
+    cap, positions = 2048, [0, 31, 32, 127, 128, 129, 1000, 2046, 2047]
+    q, kc, vc, _, run = _q8_0_batch(np.random.default_rng(hq), 9, hq, cap, positions)
+    out, bad = run(slice(0, 9), 32)
+    assert bad == 0
+    for i, p in enumerate(positions):
+        one, bad = run(slice(i, i + 1), 32)
+        assert bad == 0 and torch.equal(one[0], out[i]), p
+        k, v = kc[i * cap:(i + 1) * cap], vc[i * cap:(i + 1) * cap]
+        want, used, wbad = oracle.decode_attention_q8_0(q[i], k, v, p, local=False)
+        close, d = attn_close(out[i].cpu().numpy().view(np.uint16), want,
+                              bound_q8_0(q[i], k, v, p, False, used))
+        assert not wbad and close.all(), (p, int(d.max()))
+
+
+@pytest.mark.parametrize("seqs,splits", [(17, 1), (20, 4), (64, 4), (64, 5)])
+def test_decode_attention_q8_0_few_splits(seqs, splits):
+    """More than 16 sequences of a global cache in few splits: a workgroup per split and KV head up
+    to 64 x 4 (1024 of them), per split above.  Each sequence as alone, bit for bit, also beside
+    ones that are not admitted."""
+    print(f"[case] attention q8_0 few splits seqs={seqs} splits={splits}", flush=True)
+    cap, hq = 1024, 8
+    rng = np.random.default_rng(seqs + splits)
+    positions = rng.integers(0, cap, seqs).tolist()
+    positions[:3] = cap - 1, 0, 127
+    _, _, _, states, run = _q8_0_batch(rng, seqs, hq, cap, positions)
+    alone = torch.cat([run(slice(i, i + 1), splits)[0] for i in range(seqs)])
+    out, bad = run(slice(0, seqs), splits)
+    assert bad == 0 and torch.equal(out, alone)
+    for refused in ([0], [5, seqs - 1]):
+        some = states.clone()
+        some[refused, 7] = 1  # stopped
+        out, bad = run(slice(0, seqs), splits, some)
+        want = alone.clone()
+        want[refused] = 77
+        assert bad == 1 and torch.equal(out, want)
+
+
+@pytest.mark.parametrize("fmt", [abi.KV_BF16, abi.KV_Q8])
+@pytest.mark.parametrize("hq", [4, 32])
+def test_decode_attention_fp8_of_f32(fmt, hq):
+    """The FP8 output of fp32 activations: out, codes and scales are those of the BF16 ones, and of
+    padra_QuantizeFP8 on that row; a zero row has scale 1."""
+    print(f"[case] attention fp8 of f32 fmt={fmt} hq={hq}", flush=True)
+    seqs, cap = 5, 512
+    rng = np.random.default_rng(hq + fmt)
+    kc, vc = _rows(fmt, rng, seqs * cap), _rows(fmt, rng, seqs * cap)
+    vc[2 * cap:3 * cap] = 0
+    sc = torch.full((seqs * cap, 4, 2), 1 / 64, device="cuda")
+    kv = ops.kv_cache(fmt, torch.from_numpy(kc).cuda(), torch.from_numpy(vc).cuda(), cap, scales=sc,
+                      seq_stride=cap)
+    states = torch.tensor([[5, p, cap, 10, p, p, 0, 0] for p in (0, 33, 100, 510, 511)],
+                          dtype=torch.int32, device="cuda")
+    pos = ops.positions_decode(states, maximum=cap)
+    q = torch.from_numpy(rng.standard_normal((seqs, hq, 128)).astype(np.float32)).cuda().bfloat16()
+    got = []
+    for dtype in (torch.bfloat16, torch.float32):
+        out = torch.empty((seqs, hq, 128), dtype=dtype, device="cuda")
+        packed = torch.zeros((seqs, hq * 128), dtype=torch.uint8, device="cuda")
+        scales = torch.zeros(seqs, device="cuda")
+        bad = torch.zeros(1, dtype=torch.int32, device="cuda")
+        ops.DecodeAttention(q.to(dtype), kv, out, pos, bad, packed=packed, scales=scales)
+        again, more = torch.zeros_like(packed), torch.zeros_like(scales)
+        ops.QuantizeFP8(out.view(seqs, -1), again, more, bad)
+        assert bad.item() == 0 and torch.equal(packed, again) and torch.equal(scales, more)
+        assert scales[2].item() == 1
+        got.append((out.float(), packed, scales))
+    assert all(torch.equal(a, b) for a, b in zip(*got))
