@@ -1261,8 +1261,10 @@ KERNEL_ROLES = {
     "k_combine_norm_wide": "expert combine + residual + RMSNorm + FP8 (BF16 rows)",
     "k_attn_mx": "decode attention split (BF16 / q8 cache)",
     "k_attn_merge": "decode attention merge",
+    "k_attn_encode_fp8": "decode attention: FP8 rows of the merged output",
     "k_q8_0_query": "decode attention, q8_0 query coding",
     "k_q8_0_mx": "decode attention split (q8_0 cache)",
+    "k_q8_0_streams": "decode attention split (q8_0 cache, few workgroups)",
     "k_q8_0_mx_merge": "decode attention merge (q8_0)",
     "k_stream_copy": "streaming copy: the ceilings at each leg's byte count (mixed sizes)",
 }

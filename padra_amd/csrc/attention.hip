@@ -127,7 +127,7 @@ template <int TILE> __device__ __forceinline__ bool attn_unit(const AttnArgs &a,
 // units past the last active one are the end of the grid.  Where each sequence's
 // inactive splits (all but n / 32 of 32) came between the others' active ones, their waves, which
 // do no more than read the control records, held the slots: 64 sequences of up to 300 keys
-// (BF16) 40.4 -> 26.2 us, of up to 1000 keys (q8_0) 83.7 -> 33.9 us.
+// (BF16) 40.4 -> 18.8 us, of up to 1000 keys (q8_0) 83.7 -> 31.8 us.
 //
 // In the split kernels (2 to 16 sequences, one a lane): saves the launch of k_attn_order, 2-4 us,
 // and costs each wave 5 instructions a sequence; at 64 sequences those were 7 us of
@@ -834,9 +834,8 @@ __global__ __launch_bounds__(256) void k_attn_encode_fp8(AttnArgs a, uint8_t *pa
 // each block (fmaf in block order), then ((P0 + P1) + (P2 + P3)), times 1/sqrt(128).  Each
 // 128-key tile runs as four 32-key online-softmax streams (slice s: keys 32 s .. 32 s + 31),
 // each key lane keeping its own denominator; PV multiplies V codes by p * v_scale.  The four
-// streams join per split; the merge rotates the result back (two 64-point transforms).
-// Here (k_q8_0_mx) each stream is its own partial entry and the merge joins the 4 * splits
-// entries; scores and PV run on the matrix cores.
+// streams join per split; the merge joins the splits and rotates the result back (two 64-point
+// transforms).  Scores and PV run on the matrix cores here.
 
 // One query head's codes and block scales, by a wave: rotated features lane and lane + 64, of
 // blocks lane / 32 and 2 + lane / 32.  False (and nothing written) where a value is not finite.
@@ -1651,18 +1650,23 @@ int reference_splits(const padra_KVCache *kv, int local) {
   return std::min((kv->cap + kKeys - 1) / kKeys, local ? 16 : 32);
 }
 
-// The split count for splits = -1, from a sweep on MI355X (64-sequence decode step):
-// global windows keep the reference's count (within 1.5% of the best of 8-32); a local
-// ring's 1024-key windows want about 1,024 resident waves for BF16 and q8_0 and 2,048 for
-// q8 (1 / 8 / 64 sequences, BF16: 16 / 16 / 4 splits best; q8: 32 / 32 / 8; q8_0:
-// 16 / 16 / 4; at 64 sequences 29.4 / 23.7 / 30.2 us against 40.8 / 31.8 / 49.9 us with the
-// reference's 16).
+// The split count for splits = -1.  Global windows keep the reference's count (within 1.5% of the
+// best of 8-32 at 64 sequences).  A local ring's 1024-key windows take fewer splits the more
+// sequences there are: about 1,024 one-wave splits for BF16 and q8_0 and 2,048 for q8, which was the
+// best of a sweep when every split was one wave.  It is kept as callers' results and scratch sizes
+// follow it.  This count against the reference's 16 as the kernels are (us, 32 query heads; 1, 8, 12,
+// 24, 64 sequences):
+//   BF16   9.1 :  9.1  12.7 : 12.7  14.7 : 14.8  19.6 : 21.0  32.7 : 40.5
+//   q8    10.0 : 10.0  13.9 : 13.2  17.2 : 14.9  22.5 : 20.7  28.4 : 34.9
+//   q8_0  11.0 : 11.6  15.5 : 15.6  16.4 : 16.4  23.1 : 29.1  33.9 : 51.2
+// For q8 it is thus the slower choice from 4 to 32 sequences, as it was with one wave a split
+// (12: 17.7 : 15.2).
 int tuned_splits(const padra_KVCache *kv, int local, int seqs, int kv_heads) {
   if (!local)
     return reference_splits(kv, local);
   const int per_seq = std::max(1, seqs);
   if (kv->format == PADRA_KV_Q8_0)
-    return std::clamp(256 / per_seq, 4, 16); // one 4-wave workgroup per (split, sequence)
+    return std::clamp(256 / per_seq, 4, 16);
   const int waves = kv->format == PADRA_KV_Q8 ? 2048 : 1024;
   const int cap_splits = std::min((kv->cap + kKeys - 1) / kKeys, kv->format == PADRA_KV_Q8 ? 32 : 16);
   return std::clamp(waves / (per_seq * std::max(1, kv_heads)), std::min(2, cap_splits), cap_splits);
@@ -1791,6 +1795,11 @@ int decode_attention(void *stream, const void *q, const padra_KVCache *kv, void 
     //   4 sequences, to 8000 keys, 32 heads (512)          21.9/19.3/17.9/21.8  27.7/21.3/17.2/21.5
     //   8 sequences, the same (1024)                       27.2/25.3/27.8/36.4  29.1/24.9/25.9/36.8
     //   16 sequences, 16 heads (2048)                      36.6/37.0/43.6/62.9  32.2/34.6/38.4/64.0
+    // and on local rings, whose splits have two tiles (waves without a tile still divide PV):
+    //   1 ring, 32 heads (64)                              10.5/9.5/9.2/9.1     12.5/10.4/10.1/10.0
+    //   4 rings (256)                                      11.3/10.8/10.4/10.4  12.9/11.2/10.9/10.8
+    //   8 rings (512)                                      13.4/13.4/13.1/16.6  14.0/13.5/13.2/16.8
+    //   12 rings (768)                                     14.8/15.2/18.5/22.6  15.1/14.8/15.1/23.2
     const int wgs = splits * kv_heads * seqs;
     auto split_w = [&](auto q8tag) {
       if (wgs <= 256)
