@@ -1241,6 +1241,9 @@ KERNEL_ROLES = {
     "k_chain<128, 16, 1, false, unsigned short>": "config 2 chain, q8 KV",
     "k_chain<128, 16, 2, false, unsigned short>": "config 2 chain, q8_0 KV (rotated)",
     "k_chain<128, 16, 3, false, unsigned short>": "config 2 chain, q8_0 KV (unrotated)",
+    "k_chain<128, 16, 0, false, float>": "config 1 chain on fp32 activations, BF16 KV",
+    "k_chain<128, 18, 2, false, float>": "chain on fp32 activations, q8_0 KV (rotated)",
+    "k_chain_small<256, 9, 0, true>": "decode step, hidden 2304, BF16 KV: gather + chain",
     "k_chain_small<256, 8, 0, true>": "config 4/0 decode step: gather + chain, one launch",
     "k_chain_small<256, 8, 0, false>": "config 4/0 decode chain after a separate gather",
     "k_chain_heads<256, 8, 0, false, float>": "config 4/0 decode chain on fp32 activations, BF16 KV",
