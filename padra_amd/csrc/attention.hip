@@ -333,10 +333,11 @@ template <bool Q8> __device__ __forceinline__ int vq_slot(int d) {
 }
 
 // DENSE: for q8 launches of more one-wave workgroups than two on each SIMD (2048), held to the
-// registers of three (168 VGPRs, no spill, for 190): the decode is arithmetic, which a third wave
-// fills.  64 sequences (us): to 131072 keys (16 heads) 788 -> 727, to 32768 238 -> 222, to 8000 keys (32
-// heads) 96.9 -> 90.0; 24 to 8000 keys 50.6 -> 48.5.  In smaller launches two a SIMD is all there is
-// and the order that this takes costs 3-5%: 12 sequences to 65536 keys 154 -> 162.
+// registers of three (168 VGPRs, no spill, for 190): the decode is arithmetic, whose waits a third
+// wave fills (VALU issue 89% of the cycles then, 64 sequences to 32768 keys).  64 sequences (us): to
+// 131072 keys (16 heads) 788 -> 727, to 32768 238 -> 222, to 8000 (32 heads) 96.9 -> 90.0; 24 to
+// 8000 keys 50.6 -> 48.5.  In smaller launches two a SIMD is all there is and the order that this
+// takes costs 3-5%: 12 sequences to 65536 keys 154 -> 162.
 template <class T, bool Q8, int W, bool DENSE = false>
 __global__ __launch_bounds__(64 * W, DENSE ? 3 : 1) void k_attn_mx(AttnArgs a) {
   constexpr bool HELD = Q8 && (W > 1 || DENSE);
@@ -1654,8 +1655,8 @@ int reference_splits(const padra_KVCache *kv, int local) {
 // best of 8-32 at 64 sequences).  A local ring's 1024-key windows take fewer splits the more
 // sequences there are: about 1,024 one-wave splits for BF16 and q8_0 and 2,048 for q8, which was the
 // best of a sweep when every split was one wave.  It is kept as callers' results and scratch sizes
-// follow it.  This count against the reference's 16 as the kernels are (us, 32 query heads; 1, 8, 12,
-// 24, 64 sequences):
+// follow it.  This count against the reference's 16 as the kernels are (us, 32 query heads; 1, 8,
+// 12, 24, 64 sequences):
 //   BF16   9.1 :  9.1  12.7 : 12.7  14.7 : 14.8  19.6 : 21.0  32.7 : 40.5
 //   q8    10.0 : 10.0  13.9 : 13.2  17.2 : 14.9  22.5 : 20.7  28.4 : 34.9
 //   q8_0  11.0 : 11.6  15.5 : 15.6  16.4 : 16.4  23.1 : 29.1  33.9 : 51.2
